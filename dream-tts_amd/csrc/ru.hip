@@ -51,11 +51,12 @@ struct RuCfg {
     static constexpr int TN = C / 32;   // 32-channel blocks
     static constexpr int KMAX = 7, HMAX = 64;
     static constexpr int CHUNKS = C / KC;
-    // window: BM + HMAX rows x KC halves, rows padded by 8 halves (16 consecutive rows at one
-    // 16-byte segment then hit 16 distinct 4-bank groups)
+    // window: BM + HMAX rows x KC halves, unpadded, the segments of a row XOR-swizzled as W1's are:
+    // a wave's 16-byte writes then fill 1 KiB without a gap, and a fragment read's 32 rows spread
+    // over the banks from any starting row.
     static constexpr int ROWS = BM + HMAX;
     static constexpr int SEGS = KC / 8;
-    static constexpr int APITCH = KC + 8;
+    static constexpr int APITCH = KC;
     static constexpr int A_BYTES = ROWS * APITCH * 2;
     static constexpr int A_SEGS = ROWS * SEGS;
     static constexpr int A_PER_T = (A_SEGS + THREADS - 1) / THREADS;
@@ -146,13 +147,13 @@ __global__ __launch_bounds__(Cfg::THREADS, Cfg::WPE) void ru_nlc_f16(RuArgs q) {
         __builtin_amdgcn_make_buffer_rsrc(const_cast<half_t *>(ul), 0, q.L * C * 2, kBufferWord3);
     const int qd = tid % SEGS;
     uint32_t va[Cfg::A_PER_T];
-    int arow[Cfg::A_PER_T];
+    int aoff[Cfg::A_PER_T];
 #pragma unroll
     for (int i = 0; i < Cfg::A_PER_T; ++i) {
         const int s = i + 1 < Cfg::A_PER_T ? tid + i * Cfg::THREADS : (Cfg::A_PER_T - 1) * Cfg::THREADS + tid % LAST;
         const int r = s / SEGS;
         const int src = win0 + r;
-        arow[i] = r;
+        aoff[i] = r * APITCH * 2 + ((qd ^ seg_swizzle<KC>(r)) << 4);
         va[i] = (r < rows && src >= 0 && src < q.L) ? static_cast<uint32_t>((src * C + qd * 8) * 2) : kOutOfRange;
     }
     typedef half8_t WinRegs[Cfg::A_PER_T];
@@ -181,7 +182,7 @@ __global__ __launch_bounds__(Cfg::THREADS, Cfg::WPE) void ru_nlc_f16(RuArgs q) {
     auto win_write = [&](const WinRegs &R, char *stage) {
 #pragma unroll
         for (int i = 0; i < Cfg::A_PER_T; ++i)
-            *reinterpret_cast<half8_t *>(stage + arow[i] * APITCH * 2 + qd * 16) = R[i];
+            *reinterpret_cast<half8_t *>(stage + aoff[i]) = R[i];
     };
     auto win_store = [&](WinRegs &R, int c0, char *stage) {
         const SnakeK kk = snake_consts(c0);
@@ -229,72 +230,31 @@ __global__ __launch_bounds__(Cfg::THREADS, Cfg::WPE) void ru_nlc_f16(RuArgs q) {
                 for (int e = 0; e < 4; ++e) acc[i][j][4 * g + e] = b[e];
         }
 
-    // fragments: window (B operand) rows wave*WP + 32i + l32 + t*dil, halves hf*8; W1 (A operand)
-    // rows t*C + 32j + l32, segment hf ^ swizzle
+    // fragments: window (B operand) rows wave*WP + 32i + l32 + t*dil and W1 (A operand) rows
+    // t*C + 32j + l32, segment hf ^ swizzle
     const int prow = wave * Cfg::WP + l32;
-    // hook(t) runs in the same scheduling region as tap t's MFMAs, so its VALU work issues in
-    // their shadow
-    auto compute = [&](const char *stage, auto &&hook) {
-        const char *A = stage;
-        const char *B = stage + Cfg::A_BYTES;
-        auto frag_x = [&](int t, int i) {
-            return *reinterpret_cast<const half8_t *>(A + (prow + 32 * i + t * q.dil) * APITCH * 2 + hf * 16);
-        };
-        auto frag_w = [&](int t, int j) {
-            const int r = t * C + 32 * j + l32;
-            return *reinterpret_cast<const half8_t *>(B + r * (KC * 2) + ((hf ^ seg_swizzle<KC>(r)) << 4));
-        };
-        if constexpr (KT > 0) {
-            half8_t fx[2][TM], fw[2][TN];
+    half8_t fx[KT > 0 ? 2 : 1][TM], fw[KT > 0 ? 2 : 1][TN];  // two fragment sets when the taps are unrolled
+    auto load_frags = [&](const char *stage, int t, int set) {
+        const int r = prow + t * q.dil;  // 32 i leaves the swizzle alone
+        const char *X = stage + r * APITCH * 2 + ((hf ^ seg_swizzle<KC>(r)) << 4);
+        const char *W = stage + Cfg::A_BYTES + l32 * (KC * 2) + ((hf ^ seg_swizzle<KC>(l32)) << 4);
 #pragma unroll
-            for (int i = 0; i < TM; ++i) fx[0][i] = frag_x(0, i);
+        for (int i = 0; i < TM; ++i) fx[set][i] = *reinterpret_cast<const half8_t *>(X + 32 * i * APITCH * 2);
 #pragma unroll
-            for (int j = 0; j < TN; ++j) fw[0][j] = frag_w(0, j);
+        for (int j = 0; j < TN; ++j) fw[set][j] = *reinterpret_cast<const half8_t *>(W + (t * C + 32 * j) * (KC * 2));
+    };
+    auto mma = [&](int set) {
 #pragma unroll
-            for (int t = 0; t < KT; ++t) {
-                if (t + 1 < KT) {
+        for (int i = 0; i < TM; ++i)
 #pragma unroll
-                    for (int i = 0; i < TM; ++i) fx[(t + 1) & 1][i] = frag_x(t + 1, i);
-#pragma unroll
-                    for (int j = 0; j < TN; ++j) fw[(t + 1) & 1][j] = frag_w(t + 1, j);
-                }
-                __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-                for (int i = 0; i < TM; ++i)
-#pragma unroll
-                    for (int j = 0; j < TN; ++j)
-                        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fw[t & 1][j], fx[t & 1][i], acc[i][j], 0, 0, 0);
-                hook(t);
-                // one MFMA, then a few VALU instructions (the hook's), in turn
-#pragma unroll
-                for (int m = 0; m < TM * TN; ++m) {
-                    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-                    __builtin_amdgcn_sched_group_barrier(0x402, 4, 0);
-                }
-                __builtin_amdgcn_sched_barrier(0);
-            }
-        } else {
-            for (int t = 0; t < k; ++t) {
-                half8_t fx[TM], fw[TN];
-#pragma unroll
-                for (int i = 0; i < TM; ++i) fx[i] = frag_x(t, i);
-#pragma unroll
-                for (int j = 0; j < TN; ++j) fw[j] = frag_w(t, j);
-#pragma unroll
-                for (int i = 0; i < TM; ++i)
-#pragma unroll
-                    for (int j = 0; j < TN; ++j)
-                        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fw[j], fx[i], acc[i][j], 0, 0, 0);
-            }
-            hook(-1);
-        }
+            for (int j = 0; j < TN; ++j)
+                acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fw[set][j], fx[set][i], acc[i][j], 0, 0, 0);
     };
 
     // Pipeline. Chunk c computes from stage c & 1. During chunk c: W1 of chunk c+1 streams into
     // stage (c+1) & 1, the window of chunk c+PD into registers, and the registers holding chunk
     // c+1's window are snaked into stage (c+1) & 1. Stage (c+1) & 1 was last read by chunk c-1,
     // which every wave finished before the barrier that closed it.
-    char *stage[2] = {smem, smem + Cfg::STAGE};
     // chunk c's window in R[c % PD], loaded PD chunks ahead: three for the 192-channel unit (one
     // workgroup per CU, so no second workgroup's work covers the loads' latency), two for the
     // 96-channel one (two workgroups per CU; the registers of a third set slowed it)
@@ -311,42 +271,75 @@ __global__ __launch_bounds__(Cfg::THREADS, Cfg::WPE) void ru_nlc_f16(RuArgs q) {
                 w2r[i] = *reinterpret_cast<const half8_t *>(q.w2 + sg * 8);
         }
     };
-    w_issue(0, stage[0]);
+    w_issue(0, (smem + 0 * Cfg::STAGE));
     win_load(R[0], 0);
     if (Cfg::CHUNKS > 1) win_load(R[1], KC);
     if (PD == 3 && Cfg::CHUNKS > 2) win_load(R[PD - 1], 2 * KC);
     wait_vmem_le<(Cfg::CHUNKS > PD - 1 ? PD - 1 : Cfg::CHUNKS - 1) * Cfg::A_PER_T>();  // W1 and chunk 0's window
-    win_store(R[0], 0, stage[0]);
-    __syncthreads();
+    win_store(R[0], 0, (smem + 0 * Cfg::STAGE));
+    stage_barrier();
+    if constexpr (KT > 0) load_frags((smem + 0 * Cfg::STAGE), 0, 0);
 #pragma unroll
     for (int c = 0; c < Cfg::CHUNKS; ++c) {
         const int cur = c & 1, nxt = cur ^ 1;
-        if (c + 1 < Cfg::CHUNKS) w_issue((c + 1) * KC, stage[nxt]);
+        const bool last = c + 1 == Cfg::CHUNKS;
+        if (!last) w_issue((c + 1) * KC, (smem + nxt * Cfg::STAGE));
         if (c + PD < Cfg::CHUNKS) win_load(R[c % PD], (c + PD) * KC);
-        if (c + 1 == Cfg::CHUNKS) w2_load();
-        if (c + 1 < Cfg::CHUNKS) {
-            // the window of chunk c+1 (loaded PD-1 chunks ago; the compiler waits for those
-            // registers) is snaked in the shadow of chunk c's MFMAs
-            const SnakeK kk = snake_consts((c + 1) * KC);
-            constexpr int NE = 8 * Cfg::A_PER_T;
-            WinRegs &Rn = R[(c + 1) % PD];
-            compute(stage[cur], [&](int t) {
-                if constexpr (KT > 0) {
-                    snake_elems(Rn, kk, t * NE / KT, (t + 1) * NE / KT);
-                } else {
-                    if (t < 0) snake_elems(Rn, kk, 0, NE);
-                }
-            });
-        } else {
-            compute(stage[cur], [](int) {});
-        }
+        if (last) w2_load();
+        const SnakeK kk = snake_consts((last ? c : c + 1) * KC);
+        constexpr int NE = 8 * Cfg::A_PER_T;
+        WinRegs &Rn = R[(c + 1) % PD];
         // W1 of chunk c+1 has landed (only the newest window loads, chunk c+PD's, may be in flight)
-        if (c + PD < Cfg::CHUNKS)
-            wait_vmem_le<Cfg::A_PER_T>();
-        else if (c + 1 < Cfg::CHUNKS)
-            wait_vmem();
-        if (c + 1 < Cfg::CHUNKS) win_write(R[(c + 1) % PD], stage[nxt]);
-        stage_barrier();
+        auto wait_next = [&] {
+            if (c + PD < Cfg::CHUNKS)
+                wait_vmem_le<Cfg::A_PER_T>();
+            else if (!last)
+                wait_vmem();
+        };
+        if constexpr (KT > 0) {
+            // The taps of all chunks as one stream: tap t+1's fragments are read between tap t's MFMAs,
+            // across chunks too. The window of chunk c+1 (loaded PD-1 chunks ago) is snaked in the
+            // shadow of taps 0 .. KT-3 and written before tap KT-2's, and the chunk's one barrier sits
+            // before the last tap's MFMAs: every wave then has this chunk's last fragments in
+            // registers, and the next chunk's first ones are read under those MFMAs. With the window
+            // unpadded (its writes took 16 LDS cycles each padded, 13 now) and the reads spread between
+            // the MFMAs: 16 x 40000 x 192, 514 -> 507 us; the chip's power limit takes the rest (the
+            // tile alone: 36.7 -> 33.9 us).
+#pragma unroll
+            for (int t = 0; t < KT; ++t) {
+                const int set = (c * KT + t) & 1;
+                if (t + 2 == KT && !last) win_write(Rn, (smem + nxt * Cfg::STAGE));
+                if (t + 1 < KT) {
+                    load_frags((smem + cur * Cfg::STAGE), t + 1, set ^ 1);
+                } else {
+                    wait_next();
+                    stage_barrier();
+                    if (!last) load_frags((smem + nxt * Cfg::STAGE), 0, set ^ 1);
+                }
+                mma(set);
+                if (t + 2 < KT && !last) snake_elems(Rn, kk, t * NE / (KT - 2), (t + 1) * NE / (KT - 2));
+                // one MFMA, up to two of the next tap's fragment reads and a few VALU instructions (the
+                // snake's), in turn
+#pragma unroll
+                for (int m = 0; m < TM * TN; ++m) {
+                    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                    __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+                    __builtin_amdgcn_sched_group_barrier(0x402, 4, 0);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        } else {
+            for (int t = 0; t < k; ++t) {
+                load_frags((smem + cur * Cfg::STAGE), t, 0);
+                mma(0);
+            }
+            if (!last) {
+                snake_elems(Rn, kk, 0, NE);
+                wait_next();
+                win_write(Rn, (smem + nxt * Cfg::STAGE));
+            }
+            stage_barrier();
+        }
     }
 
     // the residual rows of this lane's positions, four channels per load (consumed at the end)
