@@ -108,36 +108,52 @@ struct Tile {
 template <int KMAX, int HMAX, typename F>
 auto with_tile(int64_t lanes, int len, int cin, int cout, bool direct, F &&f) {
     if (direct) {
-        // k <= 7 (dilated) at 96-multiples: eight waves of 64 x 96; short sequences take 256-row
-        // tiles (two workgroups per CU) so the last tile of a lane is not mostly padding
+        // k <= 7 (dilated), 32-channel steps: eight waves of 64 x 96 or 32 x 96, or four of 32 x BN when those leave
+        // most CUs without a tile (three or four stages then: a lone tile waits on its loads)
         if constexpr (KMAX == 7) {
-            if (cout % 96 == 0 && len >= 1024) return f(Tile<ConvTile<512, 96, 8, 1, 32, KMAX, HMAX, 2, kStageDirect>>{});
-            if (cout % 96 == 0) return f(Tile<ConvTile<256, 96, 4, 1, 16, KMAX, HMAX, 2, kStageDirect>>{});
+            switch (pick_tile(kTile7, kTile7Count, lanes, len, cout)) {
+                case kTile7_512x96: return f(Tile<ConvTile<512, 96, 8, 1, 32, KMAX, HMAX, 2, kStageDirect>>{});
+                case kTile7_256x96: return f(Tile<ConvTile<256, 96, 8, 1, 32, KMAX, HMAX, 2, kStageDirect>>{});
+                case kTile7_128x96: return f(Tile<ConvTile<128, 96, 4, 1, 32, KMAX, HMAX, 2, kStageDirect>>{});
+                case kTile7_128x64: return f(Tile<ConvTile<128, 64, 4, 1, 32, KMAX, HMAX, 3, kStageDirect>>{});
+                case kTile7_128x32: return f(Tile<ConvTile<128, 32, 4, 1, 32, KMAX, HMAX, 4, kStageDirect>>{});
+            }
         }
         // k = 2 (the transposed convs) at 128-multiples: 2 x 2 waves of 128 x 64 when the input is
-        // wide (cin >= 768: more matrix work per staged chunk), else 2 x 2 waves of 64 x 64; at
-        // 96-multiples four waves of 32 x 96. Two 32-channel stages: with the epilogue's plain form
-        // the smaller footprint (more workgroups per CU) beats a third stage in flight, 9% at
-        // 128 x 128 and 16% at 128 x 96 on the codec's shapes (A/B; three stages stay better for
-        // k = 1). Measured on the codec's four upsampling shapes: 10-20% over one 256 x 96 tile.
+        // wide (cin >= 768: more matrix work per staged chunk) and that fills the CUs, else 2 x 2
+        // waves of 64 x 64; 2 x 2 waves of 32 x 32 over four stages when even those leave CUs idle
+        // (1 x 25 x 1536 -> 6144: 48 -> 18 us; 4 x 250 x 4608 -> 6144, 384 tiles: 137 us on 128 x 128,
+        // 157 on 256 x 128, 203 on 64 x 64). Every tile of a k takes the same channels per step, so
+        // an output's sum has one order whatever the batch. At 96-multiples four waves of 32 x 96. Two
+        // 32-channel stages: the smaller footprint (more workgroups per CU) beats a third stage in
+        // flight, 9% at 128 x 128 and 16% at 128 x 96 on the codec's shapes.
         if constexpr (KMAX == 2) {
-            if (cout % 128 == 0 && cin >= 768) return f(Tile<ConvTile<256, 128, 2, 2, 32, KMAX, HMAX, 2, kStageDirect>>{});
+            const int64_t tiles128 = lanes * ((len + 127) / 128) * (cout / 128);
+            const int64_t tiles256 = lanes * ((len + 255) / 256) * (cout / 128);
+            if (cout % 64 == 0 && tiles128 < 192)
+                return f(Tile<ConvTile<64, 64, 2, 2, 32, KMAX, HMAX, 4, kStageDirect>>{});
+            if (cout % 128 == 0 && cin >= 768 && tiles256 >= 224)
+                return f(Tile<ConvTile<256, 128, 2, 2, 32, KMAX, HMAX, 2, kStageDirect>>{});
             if (cout % 128 == 0) return f(Tile<ConvTile<128, 128, 2, 2, 32, KMAX, HMAX, 2, kStageDirect>>{});
             if (cout % 96 == 0) return f(Tile<ConvTile<128, 96, 4, 1, 32, KMAX, HMAX, 2, kStageDirect>>{});
         }
-        // k = 1 at 128-multiples: 2 x 2 waves of 64 x 64. Three 32-channel stages in flight (three
-        // workgroups per CU) up to cin 2048; beyond, two 64-channel stages (fewer barriers per
-        // output). When that leaves fewer than 1024 tiles, 64-channel-wide tiles instead, to fill
-        // the 256 CUs. k = 1 at 192-multiples otherwise: 256 x 192 over eight waves.
+        // k = 1: 64-channel stages, two (three for the 64 x 64 tile). At few channels and many tiles
+        // the launch moves more bytes than it multiplies: three 32-channel stages and three
+        // workgroups per CU there (24 x 10000 x 384: 123 us, 130 on the 64-channel 128 x 128 tile).
         if constexpr (KMAX == 1) {
-            const int64_t tiles128 = lanes * ((len + 127) / 128) * (cout / 128);
-            if (cout % 64 == 0 && cin % 64 == 0 && (cout % 128 != 0 || tiles128 < 1024))
-                return f(Tile<ConvTile<128, 64, 2, 2, 64, KMAX, HMAX, 2, kStageDirect>>{});
-            if (cout % 128 == 0 && cin % 64 == 0 && cin > 2048)
-                return f(Tile<ConvTile<128, 128, 2, 2, 64, KMAX, HMAX, 2, kStageDirect>>{});
+            if (cout % 128 == 0 && cin < 512 && lanes * ((len + 127) / 128) * (cout / 128) >= 1024)
+                return f(Tile<ConvTile<128, 128, 2, 2, 32, KMAX, HMAX, 3, kStageDirect>>{});
+            if (cin % 64 == 0) {
+                switch (pick_tile(kTile1, kTile1Count, lanes, len, cout)) {
+                    case kTile1_256x256: return f(Tile<ConvTile<256, 256, 2, 4, 64, KMAX, HMAX, 2, kStageDirect>>{});
+                    case kTile1_256x192: return f(Tile<ConvTile<256, 192, 4, 2, 64, KMAX, HMAX, 2, kStageDirect>>{});
+                    case kTile1_128x128: return f(Tile<ConvTile<128, 128, 4, 2, 64, KMAX, HMAX, 2, kStageDirect>>{});
+                    case kTile1_128x64: return f(Tile<ConvTile<128, 64, 2, 2, 64, KMAX, HMAX, 2, kStageDirect>>{});
+                    case kTile1_64x64: return f(Tile<ConvTile<64, 64, 2, 2, 64, KMAX, HMAX, 3, kStageDirect>>{});
+                }
+            }
             if (cout % 128 == 0) return f(Tile<ConvTile<128, 128, 2, 2, 32, KMAX, HMAX, 3, kStageDirect>>{});
-            if (cout % 192 == 0 && cin % 64 == 0)
-                return f(Tile<ConvTile<256, 192, 4, 2, 64, KMAX, HMAX, 2, kStageDirect>>{});
+            if (cout % 96 == 0) return f(Tile<ConvTile<128, 96, 4, 1, 32, KMAX, HMAX, 3, kStageDirect>>{});
         }
     }
     if (cout % 96 == 0) return f(Tile<ConvTile<256, 96, 4, 1, 32, KMAX, HMAX>>{});
@@ -255,6 +271,16 @@ int conv1d_nlc_f16(const dtts_conv_desc *d, hipStream_t stream) {
     p.act = d->act;
     p.scale = d->out_scale;
 
+    // a k = 1 conv's positions are independent: the lanes as one sequence, so that a tile spans lanes
+    // instead of padding each (10 x 325 rows: 26 tiles of 128 rows, 30 lane by lane)
+    dtts_conv_desc flat = *d;
+    if (d->k == 1 && d->lanes > 1 && direct_offsets_fit(d->lanes * d->len, d->cin, d->cout, 1) &&
+        d->lanes * d->len * d->cout * 2 < (int64_t(1) << 31)) {
+        flat.len = d->lanes * d->len;
+        flat.lanes = 1;
+        p.L = static_cast<int>(flat.len);
+        d = &flat;
+    }
     const Choice ch = choose(d);
     hipError_t e;
     if (std::strcmp(ch.path, "narrow") == 0) {

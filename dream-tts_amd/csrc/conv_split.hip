@@ -179,28 +179,43 @@ struct STile {
 };
 
 // The split tiles: the f16 codec's direct-staging tiles for each class (their sweeps on the same
-// GEMM shapes), with 96-wide k = 1 tiles for the narrowest stage. Returns false when no tile
+// GEMM shapes, the reduction three times as long), with 96-wide k = 1 tiles for the narrowest stage. Returns false when no tile
 // takes the shape. cin here is K' = 3 cs; every tile's KC divides cs (KC | 3 cs and 3 is odd).
 template <int KMAX, int HMAX, typename F>
 bool with_split_tile(int64_t lanes, int len, int cin, int cout, F &&f) {
     if constexpr (KMAX == 7) {
-        if (cout % 96 == 0 && len >= 1024) return f(STile<ConvTile<512, 96, 8, 1, 32, KMAX, HMAX, 2, kStageDirect>>{}), true;
-        if (cout % 96 == 0) return f(STile<ConvTile<256, 96, 4, 1, 16, KMAX, HMAX, 2, kStageDirect>>{}), true;
+        if (cout % 96 != 0) return false;
+        switch (pick_tile(kTile7, kTile7Count, lanes, len, cout)) {
+            case kTile7_512x96: return f(STile<ConvTile<512, 96, 8, 1, 32, KMAX, HMAX, 2, kStageDirect>>{}), true;
+            case kTile7_256x96: return f(STile<ConvTile<256, 96, 8, 1, 32, KMAX, HMAX, 2, kStageDirect>>{}), true;
+            case kTile7_128x96: return f(STile<ConvTile<128, 96, 4, 1, 32, KMAX, HMAX, 2, kStageDirect>>{}), true;
+            case kTile7_128x64: return f(STile<ConvTile<128, 64, 4, 1, 32, KMAX, HMAX, 3, kStageDirect>>{}), true;
+            case kTile7_128x32: return f(STile<ConvTile<128, 32, 4, 1, 32, KMAX, HMAX, 4, kStageDirect>>{}), true;
+        }
     }
     if constexpr (KMAX == 2) {
-        if (cout % 128 == 0 && cin >= 768) return f(STile<ConvTile<256, 128, 2, 2, 32, KMAX, HMAX, 2, kStageDirect>>{}), true;
+        const int64_t tiles128 = lanes * ((len + 127) / 128) * (cout / 128);
+        const int64_t tiles256 = lanes * ((len + 255) / 256) * (cout / 128);
+        if ((cout % 128 == 0 || cout % 96 == 0) && cout % 64 == 0 && tiles128 < 192)
+            return f(STile<ConvTile<64, 64, 2, 2, 32, KMAX, HMAX, 4, kStageDirect>>{}), true;
+        if (cout % 128 == 0 && cin >= 768 && tiles256 >= 224)
+            return f(STile<ConvTile<256, 128, 2, 2, 32, KMAX, HMAX, 2, kStageDirect>>{}), true;
         if (cout % 128 == 0) return f(STile<ConvTile<128, 128, 2, 2, 32, KMAX, HMAX, 2, kStageDirect>>{}), true;
         if (cout % 96 == 0) return f(STile<ConvTile<128, 96, 4, 1, 32, KMAX, HMAX, 2, kStageDirect>>{}), true;
     }
     if constexpr (KMAX == 1) {
-        const int64_t tiles128 = lanes * ((len + 127) / 128) * (cout / 128);
         // 96 wide: 128 x 96 over four waves, three stages (three workgroups per CU; 15-23% faster
         // than 256 x 96 with two, on the codec's 96-channel k = 1 convs)
         if (cout == 96) return f(STile<ConvTile<128, 96, 4, 1, 32, KMAX, HMAX, 3, kStageDirect>>{}), true;
-        if (cout % 64 == 0 && cin % 64 == 0 && (cout % 128 != 0 || tiles128 < 1024))
-            return f(STile<ConvTile<128, 64, 2, 2, 64, KMAX, HMAX, 2, kStageDirect>>{}), true;
-        if (cout % 128 == 0 && cin % 64 == 0 && cin > 2048)
-            return f(STile<ConvTile<128, 128, 2, 2, 64, KMAX, HMAX, 2, kStageDirect>>{}), true;
+        if (cin % 64 == 0) {
+            switch (pick_tile(kTile1, kTile1Count, lanes, len, cout)) {
+                case kTile1_256x256: return f(STile<ConvTile<256, 256, 2, 4, 64, KMAX, HMAX, 2, kStageDirect>>{}), true;
+                case kTile1_256x192: return f(STile<ConvTile<256, 192, 4, 2, 64, KMAX, HMAX, 2, kStageDirect>>{}), true;
+                case kTile1_128x128: return f(STile<ConvTile<128, 128, 4, 2, 64, KMAX, HMAX, 2, kStageDirect>>{}), true;
+                case kTile1_128x64: return f(STile<ConvTile<128, 64, 2, 2, 64, KMAX, HMAX, 2, kStageDirect>>{}), true;
+                case kTile1_64x64: return f(STile<ConvTile<64, 64, 2, 2, 64, KMAX, HMAX, 3, kStageDirect>>{}), true;
+            }
+        }
         if (cout % 128 == 0) return f(STile<ConvTile<128, 128, 2, 2, 32, KMAX, HMAX, 3, kStageDirect>>{}), true;
         if (cout % 96 == 0) return f(STile<ConvTile<256, 96, 4, 1, 32, KMAX, HMAX, 2, kStageDirect>>{}), true;
     }

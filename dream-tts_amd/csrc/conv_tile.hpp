@@ -111,6 +111,49 @@ inline int pick_tiles_ng(int tiles_n, int64_t slice_bytes, int64_t budget = int6
     return best;
 }
 
+// Which tile a direct-staging conv runs on. A launch of r = tiles / 256 workgroups per CU is
+// estimated at full * floor(r), plus `light` for a last, partly filled round (a tile whose CU and
+// power budget it does not share takes `light`); the tile with the smallest estimate wins. The
+// costs are microseconds per KC-sized step of the reduction, measured over the codec's, the front
+// half's and the decoder stack's shapes at 1 to 48 lanes; the common factor, the step count,
+// is left out.
+struct TileCost {
+    int bm, bn;
+    double full, light;
+};
+
+inline double tile_cost(const TileCost &t, int64_t lanes, int64_t len, int64_t cout) {
+    const int64_t tiles = lanes * ((len + t.bm - 1) / t.bm) * (cout / t.bn);
+    const int64_t whole = tiles / 256, part = tiles % 256;
+    if (whole == 0 || tiles == 256) return whole && t.full > t.light ? t.full : t.light;
+    return static_cast<double>(whole) * t.full + (part ? t.light : 0.0);
+}
+
+// The cheapest of n tiles whose bn divides cout (-1: none does).
+inline int pick_tile(const TileCost *t, int n, int64_t lanes, int64_t len, int64_t cout) {
+    int best = -1;
+    double cost = 0.0;
+    for (int i = 0; i < n; ++i) {
+        if (cout % t[i].bn != 0) continue;
+        const double c = tile_cost(t[i], lanes, len, cout);
+        if (best < 0 || c < cost) best = i, cost = c;
+    }
+    return best;
+}
+
+// k <= 7, 32-channel steps. 24 x 2000 x 768 (three full rounds of 512 x 96): 338 us, 378 on
+// 256 x 96; 4 x 2000 x 768 over 2304 channels (128 or 256 tiles): 223 / 190; 1 x 200 x 768: 66 us on
+// 512 x 96, 43 on the 256 x 96 of four waves that short sequences took before, 16 on 128 x 32.
+enum { kTile7_512x96, kTile7_256x96, kTile7_128x96, kTile7_128x64, kTile7_128x32, kTile7Count };
+constexpr TileCost kTile7[kTile7Count] = {
+    {512, 96, 4.70, 2.70}, {256, 96, 2.62, 1.60}, {128, 96, 1.63, 1.14}, {128, 64, 1.10, 0.86}, {128, 32, 0.71, 0.67}};
+
+// k = 1, 64-channel steps. 2048 rows, 2048 -> 12288: 103 us on 256 x 192, 109 on 128 x 128, 130 on
+// 128 x 64; 701 rows, 2048 -> 2048: 16 us on 64 x 64, 24 on 128 x 128.
+enum { kTile1_256x256, kTile1_256x192, kTile1_128x128, kTile1_128x64, kTile1_64x64, kTile1Count };
+constexpr TileCost kTile1[kTile1Count] = {
+    {256, 256, 2.05, 1.65}, {256, 192, 1.60, 1.45}, {128, 128, 0.568, 0.70}, {128, 64, 0.338, 0.56}, {64, 64, 0.205, 0.35}};
+
 // Host check for direct staging: every byte offset a buffer load forms stays below 2^31, where
 // the out-of-range marker sits.
 inline bool direct_offsets_fit(int64_t len, int64_t cin, int64_t cout, int64_t k) {
