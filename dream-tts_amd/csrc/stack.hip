@@ -23,6 +23,7 @@
 // return at once). The graph is kept until a call brings other pointers or sizes.
 #include <cstring>
 #include <new>
+#include <type_traits>
 #include <vector>
 
 #include "attn.hpp"
@@ -677,234 +678,224 @@ __global__ __launch_bounds__(256) void prefill_attention(const float *q, const h
     }
 }
 
-// The same attention on the f32 matrix cores (v_mfma_f32_32x32x2_f32), one workgroup of NW
-// waves per (lane bi, head h, 32 consecutive queries ti0 ..), the waves taking alternate blocks
-// of 32 keys. A score block is K . Q^T, so a lane holds 16 keys of one query (its lane index mod
-// 32); MFMA step s pairs dimension s (lanes 0-31) with dimension D/2 + s (lanes 32-63), so a
-// lane's operands are D/2 contiguous floats of its key row and of its query row (16-byte loads).
-// The scores go to LDS ([key][query], rows 34 floats apart), masked to -inf outside each query's
-// range; then softmax_last_dim as candle computes it (max, exp(s - max), sum, probs = e / sum),
-// the waves' maxima and sums combined through LDS (the sums in wave order); then each wave's
-// out^T = V^T . P^T over its key blocks in 32-dimension blocks, two keys per step (key s and
-// s + 16 of a block), and wave 0 adds the others' partials in wave order. The dot products are summed in the matrix
-// cores' order rather than dimension order; the prefill's f32 tolerance holds either way. A
-// block's keys (or values) load under the previous block's MFMAs, within two waves per SIMD's
-// registers. LDS: the keys x 34 floats, at least (NW - 1) partial outputs of D x 32 floats.
-constexpr int kPrefillMfmaPitch = 34;          // 16 rows x 34 floats = 32 banks apart (mod 64)
-constexpr int kPrefillMfmaMaxLds = 64 * 1024;  // dynamic + static LDS; longer key ranges take prefill_attention
-constexpr int kPrefillMfmaMinT = 16;           // fewer queries leave most of a 32-query block idle
-constexpr int kPrefillMfmaWaves = 2;           // waves per 32-query block, on alternate key blocks (4: slower)
-
-// The kernel's static LDS (its `red` array of maxima and sums), counted against kPrefillMfmaMaxLds
-// with the dynamic rows.
-template <int NW>
-constexpr size_t prefill_mfma_static_lds() { return 2 * NW * 32 * sizeof(float); }
+// The same attention on the f32 matrix cores (v_mfma_f32_32x32x2_f32), for any number of keys: one
+// workgroup of NW waves per (lane bi, head h, 32 consecutive queries ti0 ..), the waves taking
+// alternate blocks of 32 keys, each with its own running softmax (max m, sum l, weighted sum o); the
+// waves' states meet in LDS at the end. Blocks hold keys of the f16 cache below start, or new f32 ones,
+// never both.
+//
+// A score block is K . Q^T, so a lane holds 16 keys (8g + 4hf + c) of one query (its index mod 32).
+// The two halves' lanes take a key row's dimensions 16 bytes in turn, so a load covers 32 contiguous
+// bytes of each row. The lane's 16 probabilities are then the operands of out^T = V^T . P^T as they
+// stand, step v pairing the two halves' v-th keys, so the scores never leave the registers; row r of
+// output block db is dimension NDB r + db, so a lane reads its dimensions of a value row in one load.
+// K's next block loads under P . V, V's under K . Q^T.
+//
+// Bound: the f32 matrix rate, 2 D / 64 MFMAs of 64 cycles per wave and block, and the longest
+// workgroup of a causal block row (long rows are dispatched first). Talker prompts, per layer: 1 x 701
+// (352 workgroups) 166 us on prefill_attention -> 53, 8 x 256 (1024) 74 us with the scores in LDS -> 50.
+constexpr int kPrefillFlashMinT = 16;    // fewer queries leave most of a 32-query block idle
+constexpr int kPrefillFlashFill = 1024;  // workgroups past which two waves each fill the chip; four below
 
 template <int D, int NW>
-__global__ __launch_bounds__(64 * NW, 2) void prefill_attention_mfma(const float *q, const half_t *kc, const half_t *vc,
-                                                                 const float *kf, const float *vf, half_t *out, int t,
-                                                                 int start, int heads, int n_kv, int cap, int window,
-                                                                 float scale) {
-#pragma clang fp contract(off)
-    extern __shared__ __attribute__((aligned(16))) float sc[];  // [keys][kPrefillMfmaPitch], then wave 1's output
-    __shared__ float red[2][NW][32];                             // [max | sum][wave][query]
-    static_assert(sizeof(red) == prefill_mfma_static_lds<NW>(), "static LDS counted on the host");
-    constexpr int H = D / 2, NDB = D / 32, P = kPrefillMfmaPitch;
+constexpr size_t prefill_flash_lds() {
+    return sizeof(float) * (NW * (D * 32 + 64) > 32 * (D + 4) ? NW * (D * 32 + 64) : 32 * (D + 4));
+}
+
+template <int D, int NW>
+__global__ __launch_bounds__(64 * NW, 2) void prefill_attention_flash(const float *q, const half_t *kc, const half_t *vc,
+                                                                     const float *kf, const float *vf, half_t *out, int t,
+                                                                     int start, int heads, int n_kv, int cap, int window,
+                                                                     float scale) {
+    constexpr int H = D / 2, NDB = D / 32, QP = D + 4;
     static_assert(D == 64 || D == 128, "head dim");
+    static_assert(16 % NW == 0, "the merge's split of the dimensions");
+    extern __shared__ __attribute__((aligned(16))) float sm[];  // the queries [32][QP]; then the waves' states
     const int w = threadIdx.x >> 6, lane = threadIdx.x & 63, l32 = lane & 31, hf = lane >> 5;
     const int qblocks = (t + 31) / 32;
-    // the query blocks of lane bi in an order rotated by bi: consecutive workgroups, which land on
-    // different CUs, mix long and short key ranges
-    const int h = blockIdx.x % heads, bi = blockIdx.x / (heads * qblocks);
-    const int qb = ((blockIdx.x / heads) % qblocks + bi) % qblocks;
+    const int per = gridDim.x / qblocks;  // lanes * heads
+    const int qb = qblocks - 1 - static_cast<int>(blockIdx.x) / per, bh = static_cast<int>(blockIdx.x) % per;
+    const int h = bh % heads, bi = bh / heads;
     const int ti0 = qb * 32;
     const int nq = t - ti0 < 32 ? t - ti0 : 32;
     const int kh = h / (heads / n_kv);
     auto lo_of = [&](int ti) { return window > 0 && start + ti + 1 > window ? start + ti + 1 - window : 0; };
-    const int lo = lo_of(ti0), hi = start + ti0 + nq - 1;  // the union of the block's key ranges
-    const int nb = (hi - lo + 32) / 32;
-    const half_t *kcr = kc + (static_cast<int64_t>(bi) * n_kv + kh) * cap * D;
-    const half_t *vcr = vc + (static_cast<int64_t>(bi) * n_kv + kh) * cap * D;
-    const float *kfr = kf + (static_cast<int64_t>(bi) * n_kv + kh) * t * D;
-    const float *vfr = vf + (static_cast<int64_t>(bi) * n_kv + kh) * t * D;
-    const bool qok = l32 < nq;
+    const int lo = lo_of(ti0), hi = start + ti0 + nq;  // the union of the block's key ranges
+    const int new0 = lo > start ? lo : start;
+    const int nbp = lo < start ? (start - lo + 31) / 32 : 0, nb = nbp + (hi - new0 + 31) / 32;
+    // a head's rows as buffers: 32-bit offsets, at most 2^14 positions (kPrefillMaxKeys)
+    auto rows_of = [&](const auto *p, int64_t head_rows, int rows) {
+        typedef typename std::remove_const<typename std::remove_pointer<decltype(p)>::type>::type E;
+        return __builtin_amdgcn_make_buffer_rsrc(const_cast<E *>(p) + (static_cast<int64_t>(bi) * n_kv + kh) * head_rows * D,
+                                                 0, rows * D * static_cast<int>(sizeof(E)), 0x00020000);
+    };
+    const __amdgpu_buffer_rsrc_t rkc = rows_of(kc, cap, start), rvc = rows_of(vc, cap, start);
+    const __amdgpu_buffer_rsrc_t rkf = rows_of(kf, t, t), rvf = rows_of(vf, t, t);
     const int tq = ti0 + l32;  // this lane's query
-    float qv[H];
+    const int key_lo = lo_of(tq), key_hi = l32 < nq ? start + tq : -1;
     {
-        const float *qr = q + ((static_cast<int64_t>(bi) * heads + h) * t + (qok ? tq : ti0)) * D + hf * H;
-#pragma unroll
-        for (int e = 0; e < H; e += 4) {
-            const float4_t v = *reinterpret_cast<const float4_t *>(qr + e);
-#pragma unroll
-            for (int c = 0; c < 4; ++c) qv[e + c] = qok ? v[c] : 0.0f;
+        const float *qr = q + ((static_cast<int64_t>(bi) * heads + h) * t + ti0) * D;
+        for (int e = threadIdx.x * 4; e < 32 * D; e += 64 * NW * 4) {
+            const int r = e / D, d = e % D;
+            *reinterpret_cast<float4_t *>(sm + r * QP + d) =
+                r < nq ? *reinterpret_cast<const float4_t *>(qr + r * D + d) : float4_t{0.f, 0.f, 0.f, 0.f};
         }
     }
-    // key row j's dims hf*H .. hf*H + H - 1 as f32 (zeros past the range)
-    auto load_k = [&](int j, float (&kv)[H]) {
-        if (j > hi) {
+    // The wave's blocks b0, b0 + NW, .. < b1 of one kind (PRIOR: the cache's rows), block b holding keys
+    // base + 32 b ..; rows past `end` repeat the last one and are masked.
+    auto load_k = [&](auto prior, int j0, int end, float (&kv)[H]) {
+        const int j = j0 + l32 < end ? j0 + l32 : end - 1;
+        if constexpr (decltype(prior)::value) {
+            const int off = (j * D + 8 * hf) * 2;
 #pragma unroll
-            for (int e = 0; e < H; ++e) kv[e] = 0.0f;
-        } else if (j < start) {
-            const half_t *kr = kcr + static_cast<int64_t>(j) * D + hf * H;
+            for (int d = 0; d < H; d += 8) {
+                const half8_t v = __builtin_bit_cast(half8_t, __builtin_amdgcn_raw_buffer_load_b128(rkc, off + d * 4, 0, 0));
 #pragma unroll
-            for (int e = 0; e < H; e += 8) {
-                const half8_t v = *reinterpret_cast<const half8_t *>(kr + e);
-#pragma unroll
-                for (int c = 0; c < 8; ++c) kv[e + c] = static_cast<float>(v[c]);
+                for (int c = 0; c < 8; ++c) kv[d + c] = static_cast<float>(v[c]);
             }
         } else {
-            const float *kr = kfr + static_cast<int64_t>(j - start) * D + hf * H;
+            const int off = ((j - start) * D + 4 * hf) * 4;
 #pragma unroll
-            for (int e = 0; e < H; e += 4) {
-                const float4_t v = *reinterpret_cast<const float4_t *>(kr + e);
+            for (int d = 0; d < H; d += 4) {
+                const float4_t v = __builtin_bit_cast(float4_t, __builtin_amdgcn_raw_buffer_load_b128(rkf, off + d * 8, 0, 0));
 #pragma unroll
-                for (int c = 0; c < 4; ++c) kv[e + c] = v[c];
+                for (int c = 0; c < 4; ++c) kv[d + c] = v[c];
             }
         }
     };
-    float mx = -INFINITY;  // over this lane's rows of its query's scores
-    auto score_block = [&](int b, const float (&kv)[H]) {
-        float16_t acc = {};
-#pragma unroll
-        for (int s = 0; s < H; ++s) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(kv[s], qv[s], acc, 0, 0, 0);
+    // a lane's NDB dimensions NDB * l32 .. of each of its 16 keys
+    auto load_v = [&](auto prior, int j0, int end, float (&vv)[16][NDB]) {
 #pragma unroll
         for (int v = 0; v < 16; ++v) {
-            const int i = 32 * b + 8 * (v >> 2) + 4 * hf + (v & 3);  // key lo + i
-            const int jj = lo + i;
-            const bool in = qok && jj <= start + tq && jj >= lo_of(tq);
-            float x = acc[v];
-            if (scale != 1.0f) x = x * scale;
-            sc[i * P + l32] = in ? x : -INFINITY;
-            if (in) mx = fmaxf(mx, x);
-        }
-    };
-    {
-        // the wave's blocks w, w + 2, ...: the next one's keys load under the current one's MFMAs
-        float k0[H], k1[H];
-        if (w < nb) load_k(lo + 32 * w + l32, k0);
-        for (int b = w; b < nb; b += 2 * NW) {
-            if (b + NW < nb) load_k(lo + 32 * (b + NW) + l32, k1);
-            score_block(b, k0);
-            if (b + NW < nb) {
-                if (b + 2 * NW < nb) load_k(lo + 32 * (b + 2 * NW) + l32, k0);
-                score_block(b + NW, k1);
+            const int jj = j0 + 4 * hf + 8 * (v >> 2) + (v & 3), j = jj < end ? jj : end - 1;
+            if constexpr (decltype(prior)::value) {
+                typedef half_t hv_t __attribute__((ext_vector_type(NDB)));
+                const int off = (j * D + NDB * l32) * 2;
+                hv_t x;
+                if constexpr (NDB == 4)
+                    x = __builtin_bit_cast(hv_t, __builtin_amdgcn_raw_buffer_load_b64(rvc, off, 0, 0));
+                else
+                    x = __builtin_bit_cast(hv_t, __builtin_amdgcn_raw_buffer_load_b32(rvc, off, 0, 0));
+#pragma unroll
+                for (int db = 0; db < NDB; ++db) vv[v][db] = static_cast<float>(x[db]);
+            } else {
+                typedef float fv_t __attribute__((ext_vector_type(NDB)));
+                const int off = ((j - start) * D + NDB * l32) * 4;
+                fv_t x;
+                if constexpr (NDB == 4)
+                    x = __builtin_bit_cast(fv_t, __builtin_amdgcn_raw_buffer_load_b128(rvf, off, 0, 0));
+                else
+                    x = __builtin_bit_cast(fv_t, __builtin_amdgcn_raw_buffer_load_b64(rvf, off, 0, 0));
+#pragma unroll
+                for (int db = 0; db < NDB; ++db) vv[v][db] = x[db];
             }
         }
-    }
-    // softmax over the query's keys: each wave over its own blocks' rows, lane (query l32, half
-    // hf) taking every second row; the waves' maxima and sums meet in LDS
-    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-    if (hf == 0) red[0][w][l32] = mx;
-    __syncthreads();
-    mx = red[0][0][l32];
-#pragma unroll
-    for (int u = 1; u < NW; ++u) mx = fmaxf(mx, red[0][u][l32]);
-    float sum = 0.0f;
-    for (int b = w; b < nb; b += NW)
-        for (int r = hf; r < 32; r += 2) {
-            const int i = 32 * b + r;
-            const float e = qok ? expf(sc[i * P + l32] - mx) : 0.0f;  // exactly 0 outside the range
-            sc[i * P + l32] = e;
-            sum += e;
-        }
-    sum += __shfl_xor(sum, 32, 64);
-    if (hf == 0) red[1][w][l32] = sum;
-    __syncthreads();
-    sum = red[1][0][l32];
-#pragma unroll
-    for (int u = 1; u < NW; ++u) sum += red[1][u][l32];  // in wave order
-    for (int b = w; b < nb; b += NW)
-        for (int r = hf; r < 32; r += 2) {
-            const int i = 32 * b + r;
-            sc[i * P + l32] = qok ? sc[i * P + l32] / sum : 0.0f;
-        }
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // the wave's probabilities, read by its lanes below
-    __builtin_amdgcn_wave_barrier();
-    // out^T[d][query] = sum over the wave's keys of v[key][d] p[query][key]; lane: dimension l32
-    // of each 32-dimension block
+    };
+    const float s2 = scale * 1.44269504088896341f;  // scores in base 2
+    float m = -INFINITY, l = 0.0f;
     float16_t o[NDB];
 #pragma unroll
     for (int db = 0; db < NDB; ++db) o[db] = float16_t{};
-    auto load_v = [&](int b, float (&vv)[NDB][16]) {
+    __syncthreads();  // the queries
+    const float *qs = sm + l32 * QP;
+    auto run = [&](auto prior, int b0, int b1, int base, int end) {
+        if (b0 >= b1) return;
+        float kv[H], vv[16][NDB];
+        load_k(prior, base + 32 * b0, end, kv);
+        for (int b = b0; b < b1; b += NW) {
+            const int j0 = base + 32 * b;
+            load_v(prior, j0, end, vv);
+            float16_t s = {};
 #pragma unroll
-        for (int s = 0; s < 16; ++s) {
-            const int j = lo + 32 * b + s + 16 * hf;
-            if (j > hi) {
+            for (int d = 0; d < H; d += 4) {
+                // the dimensions of k's operands d .. d + 3: 8 (cache) or 4 (new) per half in turn
+                const float4_t q4 = *reinterpret_cast<const float4_t *>(
+                    qs + (decltype(prior)::value ? 2 * (d & ~7) + 8 * hf + (d & 4) : 2 * d + 4 * hf));
 #pragma unroll
-                for (int db = 0; db < NDB; ++db) vv[db][s] = 0.0f;
-            } else if (j < start) {
-                const half_t *vr = vcr + static_cast<int64_t>(j) * D + l32;
-#pragma unroll
-                for (int db = 0; db < NDB; ++db) vv[db][s] = static_cast<float>(vr[32 * db]);
-            } else {
-                const float *vr = vfr + static_cast<int64_t>(j - start) * D + l32;
-#pragma unroll
-                for (int db = 0; db < NDB; ++db) vv[db][s] = vr[32 * db];
+                for (int c = 0; c < 4; ++c) s = __builtin_amdgcn_mfma_f32_32x32x2f32(kv[d + c], q4[c], s, 0, 0, 0);
             }
+            load_k(prior, j0 + 32 * NW, end, kv);  // past the last block: its last row again, unused
+            float mx = m;
+#pragma unroll
+            for (int v = 0; v < 16; ++v) {
+                const int j = j0 + 4 * hf + 8 * (v >> 2) + (v & 3);
+                s[v] = j < end && j >= key_lo && j <= key_hi ? s[v] * s2 : -INFINITY;
+                mx = fmaxf(mx, s[v]);
+            }
+            mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+            const float mu = mx == -INFINITY ? 0.0f : mx;  // a query that has seen no key yet keeps zeros
+            const float c = __builtin_amdgcn_exp2f(m - mu);
+            m = mx;
+            float sum = 0.0f;
+#pragma unroll
+            for (int v = 0; v < 16; ++v) {
+                s[v] = __builtin_amdgcn_exp2f(s[v] - mu);
+                sum += s[v];
+            }
+            l = l * c + sum;
+#pragma unroll
+            for (int db = 0; db < NDB; ++db) o[db] = o[db] * c;
+#pragma unroll
+            for (int v = 0; v < 16; ++v)
+#pragma unroll
+                for (int db = 0; db < NDB; ++db) o[db] = __builtin_amdgcn_mfma_f32_32x32x2f32(vv[v][db], s[v], o[db], 0, 0, 0);
         }
     };
-    auto pv_block = [&](int b, const float (&vv)[NDB][16]) {
-#pragma unroll
-        for (int s = 0; s < 16; ++s) {
-            const float p = sc[(32 * b + s + 16 * hf) * P + l32];
-#pragma unroll
-            for (int db = 0; db < NDB; ++db) o[db] = __builtin_amdgcn_mfma_f32_32x32x2f32(vv[db][s], p, o[db], 0, 0, 0);
-        }
-    };
-    {
-        float v0[NDB][16], v1[NDB][16];
-        if (w < nb) load_v(w, v0);
-        for (int b = w; b < nb; b += 2 * NW) {
-            if (b + NW < nb) load_v(b + NW, v1);
-            pv_block(b, v0);
-            if (b + NW < nb) {
-                if (b + 2 * NW < nb) load_v(b + 2 * NW, v0);
-                pv_block(b + NW, v1);
-            }
-        }
-    }
-    // the other waves' partials to LDS once every wave is done with the probabilities; wave 0 adds
-    // them in wave order
-    __syncthreads();
-    if (w > 0) {
-        float *mine = sc + (w - 1) * D * 32;
-#pragma unroll
-        for (int db = 0; db < NDB; ++db)
-#pragma unroll
-            for (int v = 0; v < 16; ++v) mine[(db * 16 + v) * 64 + lane] = o[db][v];
-    }
-    __syncthreads();
-    if (w > 0 || !qok) return;
-#pragma unroll
-    for (int u = 1; u < NW; ++u) {
-        const float *part = sc + (u - 1) * D * 32;
-#pragma unroll
-        for (int db = 0; db < NDB; ++db)
-#pragma unroll
-            for (int v = 0; v < 16; ++v) o[db][v] = o[db][v] + part[(db * 16 + v) * 64 + lane];
-    }
-    half_t *dst = out + (static_cast<int64_t>(bi) * t + tq) * heads * D + h * D;
+    // block b of the wave: every NW-th over both kinds
+    run(std::true_type{}, w, nbp, lo, start);
+    run(std::false_type{}, (w - nbp % NW + NW) % NW, nb - nbp, new0, hi);
+    // the waves' states: out = sum_w o_w 2^(m_w - M) / sum_w l_w 2^(m_w - M), in wave order; each wave
+    // finishes its share of the dimensions
+    l += __shfl_xor(l, 32, 64);
+    __syncthreads();  // the queries are read
+    float *os = sm, *ms = sm + NW * D * 32, *ls = ms + NW * 32;
 #pragma unroll
     for (int db = 0; db < NDB; ++db)
 #pragma unroll
-        for (int g = 0; g < 4; ++g) {
-            half4_t r;
+        for (int v = 0; v < 16; ++v) os[((w * NDB + db) * 16 + v) * 64 + lane] = o[db][v];
+    if (hf == 0) {
+        ms[w * 32 + l32] = m;
+        ls[w * 32 + l32] = l;
+    }
+    __syncthreads();
+    if (l32 >= nq) return;
+    float mt = -INFINITY, den = 0.0f, f[NW];
 #pragma unroll
-            for (int c = 0; c < 4; ++c) r[c] = static_cast<half_t>(o[db][4 * g + c]);
-            *reinterpret_cast<half4_t *>(dst + 32 * db + 8 * g + 4 * hf) = r;
+    for (int u = 0; u < NW; ++u) mt = fmaxf(mt, ms[u * 32 + l32]);
+#pragma unroll
+    for (int u = 0; u < NW; ++u) {
+        f[u] = __builtin_amdgcn_exp2f(ms[u * 32 + l32] - mt);  // 0 for a wave that saw no key of the query
+        den += ls[u * 32 + l32] * f[u];
+    }
+    half_t *dst = out + (static_cast<int64_t>(bi) * t + tq) * heads * D + h * D;
+    typedef half_t hv_t __attribute__((ext_vector_type(NDB)));
+#pragma unroll
+    for (int i = 0; i < 16 / NW; ++i) {
+        const int v = w * (16 / NW) + i;
+        hv_t r;
+#pragma unroll
+        for (int db = 0; db < NDB; ++db) {
+            float num = 0.0f;
+#pragma unroll
+            for (int u = 0; u < NW; ++u) num += os[((u * NDB + db) * 16 + v) * 64 + lane] * f[u];
+            r[db] = static_cast<half_t>(num / den);
         }
+        *reinterpret_cast<hv_t *>(dst + NDB * (8 * (v >> 2) + 4 * hf + (v & 3))) = r;
+    }
 }
 
-// The largest key range of any 32-query block of a prefill (prefill_attention_mfma's LDS rows).
-int prefill_block_keys(int t, int start, int window) {
-    int most = 0;
-    for (int ti0 = 0; ti0 < t; ti0 += 32) {
-        const int nq = t - ti0 < 32 ? t - ti0 : 32;
-        const int lo = window > 0 && start + ti0 + 1 > window ? start + ti0 + 1 - window : 0;
-        const int n = start + ti0 + nq - lo;
-        most = n > most ? n : most;
-    }
-    return most;
+template <int D>
+hipError_t launch_prefill_flash(const float *q, const half_t *kc, const half_t *vc, const float *kf, const float *vf,
+                                half_t *out, int lanes, int t, int start, int heads, int n_kv, int cap, int window,
+                                float scale, hipStream_t stream) {
+    const unsigned blocks = static_cast<unsigned>(lanes * ((t + 31) / 32) * heads);
+    if (blocks >= kPrefillFlashFill)
+        prefill_attention_flash<D, 2><<<blocks, 128, prefill_flash_lds<D, 2>(), stream>>>(q, kc, vc, kf, vf, out, t, start, heads,
+                                                                                        n_kv, cap, window, scale);
+    else
+        prefill_attention_flash<D, 4><<<blocks, 256, prefill_flash_lds<D, 4>(), stream>>>(q, kc, vc, kf, vf, out, t, start, heads,
+                                                                                        n_kv, cap, window, scale);
+    return hipGetLastError();
 }
 
 // Up to this many rows the prefill's projections run on the A-sharing kernel (its k ranges keep
@@ -1016,16 +1007,8 @@ int enqueue_prefill(const dtts_stack &s, const float *x, float *out, const dtts_
     const int per_wave = (keys + hd) * 4 * qp;  // LDS bytes: the scores and the queries
     const int wpb = per_wave * 4 <= 65536 ? 4 : (per_wave * 2 <= 65536 ? 2 : 1);
     const int att_waves = lanes * ((t + qp - 1) / qp) * heads;
-    // 32-query blocks on the matrix cores when there are enough queries and every block's keys
-    // fit its LDS
-    const size_t mfma_lds = static_cast<size_t>((prefill_block_keys(t, start, static_cast<int>(g.window)) + 31) / 32) *
-                            32 * kPrefillMfmaPitch * sizeof(float);
-    const size_t mfma_parts = static_cast<size_t>(kPrefillMfmaWaves - 1) * hd * 32 * sizeof(float);  // waves 1.. partials
-    const size_t mfma_lds_launch = mfma_lds > mfma_parts ? mfma_lds : mfma_parts;
-    // the whole workgroup's LDS within 64 KB: 14 key blocks (448 keys) at most
-    const bool attn_mfma = t >= kPrefillMfmaMinT && (hd == 64 || hd == 128) &&
-                           mfma_lds_launch + prefill_mfma_static_lds<kPrefillMfmaWaves>() <= kPrefillMfmaMaxLds;
-    const unsigned mfma_blocks = static_cast<unsigned>(lanes * ((t + 31) / 32) * heads);
+    // 32-query blocks on the matrix cores when there are enough queries
+    const bool attn_mfma = t >= kPrefillFlashMinT;
     Partials pending{};
     const half_t *pending16 = nullptr;
     bool pending_round = false;
@@ -1058,12 +1041,9 @@ int enqueue_prefill(const dtts_stack &s, const float *x, float *out, const dtts_
 #define DTTS_PREFILL_ATTN(D_, QP_)                                                                                   \
     prefill_attention<D_, QP_><<<at_blocks, 256, lds, stream>>>(q, kc, vc, kf, vf, a16, lanes, t, start, heads, n_kv, \
                                                                  cap, static_cast<int>(g.window), scale, keys, wpb)
-        if (attn_mfma && hd == 128) {
-            prefill_attention_mfma<128, kPrefillMfmaWaves><<<mfma_blocks, 64 * kPrefillMfmaWaves, mfma_lds_launch, stream>>>(
-                q, kc, vc, kf, vf, a16, t, start, heads, n_kv, cap, static_cast<int>(g.window), scale);
-        } else if (attn_mfma) {
-            prefill_attention_mfma<64, kPrefillMfmaWaves><<<mfma_blocks, 64 * kPrefillMfmaWaves, mfma_lds_launch, stream>>>(
-                q, kc, vc, kf, vf, a16, t, start, heads, n_kv, cap, static_cast<int>(g.window), scale);
+        if (attn_mfma) {
+            PREFILL_STEP((hd == 128 ? launch_prefill_flash<128> : launch_prefill_flash<64>)(
+                q, kc, vc, kf, vf, a16, lanes, t, start, heads, n_kv, cap, static_cast<int>(g.window), scale, stream));
         } else if (hd == 128) {
             if (qp == 4)
                 DTTS_PREFILL_ATTN(128, 4);

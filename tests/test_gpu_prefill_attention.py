@@ -1,0 +1,40 @@
+"""The prefill's 32-query attention blocks at their edges, against the oracle with the prefill's bars
+(outputs 5e-4, written cache entries 1e-3): query counts around a block, key ranges that end inside a
+32-key block of either kind (the cache's rows, the new ones), windows that mask whole blocks for some
+of a block's queries, and both wave counts of the launch rule (two waves from 1024 workgroups on)."""
+from dataclasses import replace
+
+import pytest
+import torch
+
+import oracle
+from dtts import stack, synth
+
+from _stack_ref import SMALL, WINDOWED, inputs
+from _util import rel, to_dev, to_host
+
+pytestmark = pytest.mark.gpu
+
+LONG = replace(SMALL, layers=1, capacity=1024)
+WIN = replace(WINDOWED, layers=1, window=40, capacity=1024)
+
+
+@pytest.mark.parametrize("geo,lanes,t,start", [
+    (LONG, 1, 16, 0), (LONG, 2, 31, 1), (LONG, 1, 32, 31), (LONG, 2, 33, 32), (LONG, 1, 65, 33), (LONG, 1, 129, 700),
+    (LONG, 1, 500, 0), (WIN, 1, 16, 0), (WIN, 2, 45, 39), (WIN, 1, 100, 41), (WIN, 1, 300, 500), (LONG, 40, 200, 5),
+])
+def test_prefill_attention_blocks(dev, geo, lanes, t, start):
+    layers, fn = stack.random_weights(geo, 7)
+    cap = start + t
+    _, kc, vc = inputs(geo, 7, lanes, cap)
+    x = synth.normal(7, "prefill.x", (lanes, t, geo.dim))
+    st = stack.Stack(geo, layers, fn, dev)
+    state = st.new_state(lanes, cap)
+    state.k[0].copy_(to_dev(kc[0], dev))
+    state.v[0].copy_(to_dev(vc[0], dev))
+    want = oracle.stack_prefill_f32(geo, layers, fn, x, kc, vc, start)
+    got = to_host(st.prefill(to_dev(x, dev), state, start))
+    torch.cuda.synchronize()
+    assert rel(got, want)[1] < 5e-4, rel(got, want)
+    for g, w in ((state.k[0], kc[0]), (state.v[0], vc[0])):
+        assert rel(synth.from_f16_bits(to_host(g)), synth.from_f16_bits(w))[1] < 1e-3
