@@ -37,13 +37,11 @@ int decode_attention(const char *name, const float *q, const T *kc, const T *vc,
     // split the spans when a workspace holds every chunk's state (and there is more than one)
     const size_t need = attn_workspace_bytes(b, n_kv, gqa, head_dim, max_window);
     float *part = nullptr;
-    int max_chunks = 0;
     if (need > 0 && workspace && ws_bytes >= need) {
         DTTS_REQUIRE(aligned(workspace, 16), "%s: misaligned workspace", name);
         part = static_cast<float *>(workspace);
-        max_chunks = static_cast<int>((max_window + kChunk - 1) / kChunk);
     }
-    const hipError_t e = launch_attention(q, kc, vc, out, part, max_chunks, b, n_kv, gqa, head_dim, cap, sp, stream);
+    const hipError_t e = launch_attention(q, kc, vc, out, part, static_cast<int>(max_window), kChunk, b, n_kv, gqa, head_dim, cap, sp, stream);
     DTTS_HIP_CHECK(e, name);
     return DTTS_OK;
 }

@@ -110,19 +110,30 @@ __device__ __forceinline__ float group16_sum(float v) {
 constexpr float kLog2e = 1.44269504088896340736f;
 __device__ __forceinline__ float softmax_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 
-constexpr int kChunk = 512;  // positions per workgroup when a span is split
+// Positions per workgroup when a span is split: kChunk at the entry points, whose workspace sizes
+// are part of their interface. The stack step, which owns its workspace, halves it down to kChunkMin
+// while the launch has fewer than three workgroups per CU: a workgroup is a chain of dependent
+// softmax updates, and few lanes leave most CUs without one. 8 lanes, f32 caches of 1536 positions:
+// 28.8 -> 15.3 us a layer, the merge 4.8 -> 5.3.
+constexpr int kChunk = 512, kChunkMin = 128, kChunkFill = 768;
+
+inline int attn_step_chunk(int64_t b, int64_t n_kv, int64_t max_window) {
+    int c = kChunk;
+    while (c > kChunkMin && b * n_kv * ((max_window + c - 1) / c) < kChunkFill) c /= 2;
+    return c < 2 * kChunkMin && max_window <= 2 * kChunkMin ? 2 * kChunkMin : c;  // a short window stays whole
+}
 
 // Chunks of a lane's window [lo, hi) when split.
-__device__ __host__ inline int chunks_of(int lo, int hi) { return (hi - lo + kChunk - 1) / kChunk; }
+__device__ __host__ inline int chunks_of(int lo, int hi, int chunk) { return (hi - lo + chunk - 1) / chunk; }
 
 // T: cache element type; D: head dim (64 or 128); GQA: query heads per kv head; NW: waves;
 // Src: HostSpans or DevSpans; OutT: float, or half_t for a consumer that casts the result.
 // part == nullptr: blockIdx.y is 0 and the workgroup writes out. Otherwise blockIdx.y is a chunk
-// of kChunk positions, and the workgroup writes its state to part (rows of D + 2 floats: the
+// of `chunk` positions, and the workgroup writes its state to part (rows of D + 2 floats: the
 // weighted v sum, the weight sum, the max score) at [(bh * max_chunks + chunk) * GQA + g].
 template <typename T, int D, int GQA, int NW, typename Src, typename OutT>
 __global__ __launch_bounds__(NW * 64) void decode_attn_kernel(const float *q, const T *kc, const T *vc, OutT *out,
-                                                              float *part, int max_chunks, int n_kv, int cap,
+                                                              float *part, int max_chunks, int chunk, int n_kv, int cap,
                                                               Src sp) {
     constexpr int E = D / 16;     // dimensions per lane
     constexpr int G = NW * 4;     // position groups
@@ -138,9 +149,9 @@ __global__ __launch_bounds__(NW * 64) void decode_attn_kernel(const float *q, co
     int lo, hi;
     sp.get(lane_idx, lo, hi);
     if (part) {
-        if (static_cast<int>(blockIdx.y) >= chunks_of(lo, hi)) return;  // the whole workgroup
-        lo += blockIdx.y * kChunk;
-        hi = hi < lo + kChunk ? hi : lo + kChunk;
+        if (static_cast<int>(blockIdx.y) >= chunks_of(lo, hi, chunk)) return;  // the whole workgroup
+        lo += blockIdx.y * chunk;
+        hi = hi < lo + chunk ? hi : lo + chunk;
     }
 
     float qv[GQA][E];
@@ -278,47 +289,46 @@ __global__ __launch_bounds__(NW * 64) void decode_attn_kernel(const float *q, co
 // Merges the chunk states of each (lane, kv head): out = sum_c num_c e^(m_c - M) / sum_c den_c
 // e^(m_c - M), M the largest m_c, chunks in order (m in log2 units, so 2^(m_c - M)).
 template <int D, int GQA, typename Src, typename OutT>
-__global__ __launch_bounds__(256) void decode_attn_merge(const float *part, OutT *out, int max_chunks, int n_kv,
-                                                         Src sp) {
+__global__ __launch_bounds__(256) void decode_attn_merge(const float *part, OutT *out, int max_chunks, int chunk,
+                                                         int n_kv, Src sp) {
     const int bh = blockIdx.x;
     const int lane_idx = bh / n_kv;
     int lo, hi;
     sp.get(lane_idx, lo, hi);
-    const int nch = chunks_of(lo, hi);
-    constexpr int U = 8;  // chunk states requested together (a loop would wait for each in turn)
+    const int nch = chunks_of(lo, hi, chunk);
+    constexpr int U = 16;  // chunk states requested together (a loop would wait for each in turn)
     for (int t = threadIdx.x; t < GQA * D; t += 256) {
         const int g = t / D, d = t - (t / D) * D;
         const float *pr = part + (static_cast<int64_t>(bh) * max_chunks * GQA + g) * (D + 2);
         const int64_t stride = static_cast<int64_t>(GQA) * (D + 2);
-        float num = 0.0f, den = 0.0f;
-        if (nch <= U) {
+        float num = 0.0f, den = 0.0f, m = -INFINITY;
+        for (int c0 = 0; c0 < nch; c0 += U) {
             float mc[U], nc[U], dc[U];
 #pragma unroll
             for (int c = 0; c < U; ++c)
-                if (c < nch) {
-                    mc[c] = pr[c * stride + D + 1];
-                    nc[c] = pr[c * stride + d];
-                    dc[c] = pr[c * stride + D];
+                if (c0 + c < nch) {
+                    const float *pc = pr + (c0 + c) * stride;
+                    mc[c] = pc[D + 1];
+                    nc[c] = pc[d];
+                    dc[c] = pc[D];
                 }
-            float mx = -INFINITY;
+            float mx = m;
 #pragma unroll
             for (int c = 0; c < U; ++c)
-                if (c < nch) mx = fmaxf(mx, mc[c]);
+                if (c0 + c < nch) mx = fmaxf(mx, mc[c]);
+            if (c0 > 0) {  // the sums so far, at the new maximum
+                const float f = softmax_exp2(m - mx);
+                num *= f;
+                den *= f;
+            }
+            m = mx;
 #pragma unroll
             for (int c = 0; c < U; ++c)
-                if (c < nch) {
+                if (c0 + c < nch) {
                     const float f = softmax_exp2(mc[c] - mx);
                     num += nc[c] * f;
                     den += dc[c] * f;
                 }
-        } else {
-            float mx = -INFINITY;
-            for (int c = 0; c < nch; ++c) mx = fmaxf(mx, pr[c * stride + D + 1]);
-            for (int c = 0; c < nch; ++c) {
-                const float f = softmax_exp2(pr[c * stride + D + 1] - mx);
-                num += pr[c * stride + d] * f;
-                den += pr[c * stride + D] * f;
-            }
         }
         store_out(out + (static_cast<int64_t>(bh) * GQA + g) * D + d, num / den);
     }
@@ -336,49 +346,51 @@ constexpr size_t attn_lds_pad() {
 }
 
 template <typename T, int D, int GQA, typename Src, typename OutT>
-hipError_t launch_gqa(const float *q, const T *kc, const T *vc, OutT *out, float *part, int max_chunks, int64_t b,
+hipError_t launch_gqa(const float *q, const T *kc, const T *vc, OutT *out, float *part, int max_chunks, int chunk, int64_t b,
                       int64_t n_kv, int64_t cap, const Src &sp, hipStream_t stream) {
     const unsigned grid = static_cast<unsigned>(b * n_kv);
     constexpr size_t pad = attn_lds_pad<T, D, GQA>();
     if (!part) {
         decode_attn_kernel<T, D, GQA, 4, Src, OutT><<<grid, 256, pad, stream>>>(
-            q, kc, vc, out, nullptr, 0, static_cast<int>(n_kv), static_cast<int>(cap), sp);
+            q, kc, vc, out, nullptr, 0, 0, static_cast<int>(n_kv), static_cast<int>(cap), sp);
         return hipGetLastError();
     }
     decode_attn_kernel<T, D, GQA, 4, Src, OutT><<<dim3(grid, max_chunks), 256, pad, stream>>>(
-        q, kc, vc, out, part, max_chunks, static_cast<int>(n_kv), static_cast<int>(cap), sp);
+        q, kc, vc, out, part, max_chunks, chunk, static_cast<int>(n_kv), static_cast<int>(cap), sp);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    decode_attn_merge<D, GQA, Src, OutT><<<grid, 256, 0, stream>>>(part, out, max_chunks, static_cast<int>(n_kv), sp);
+    decode_attn_merge<D, GQA, Src, OutT><<<grid, 256, 0, stream>>>(part, out, max_chunks, chunk, static_cast<int>(n_kv), sp);
     return hipGetLastError();
 }
 
 // gqa in {1, 2, 4, 8} and D in {64, 128}, checked by the caller.
 template <typename T, typename Src, typename OutT>
-hipError_t launch_attention(const float *q, const T *kc, const T *vc, OutT *out, float *part, int max_chunks,
-                            int64_t b, int64_t n_kv, int64_t gqa, int64_t head_dim, int64_t cap, const Src &sp,
+hipError_t launch_attention(const float *q, const T *kc, const T *vc, OutT *out, float *part, int max_window,
+                            int chunk, int64_t b, int64_t n_kv, int64_t gqa, int64_t head_dim, int64_t cap, const Src &sp,
                             hipStream_t stream) {
+    const int max_chunks = part ? (max_window + chunk - 1) / chunk : 0;
     if (head_dim == 128) {
         switch (gqa) {
-            case 1: return launch_gqa<T, 128, 1>(q, kc, vc, out, part, max_chunks, b, n_kv, cap, sp, stream);
-            case 2: return launch_gqa<T, 128, 2>(q, kc, vc, out, part, max_chunks, b, n_kv, cap, sp, stream);
-            case 4: return launch_gqa<T, 128, 4>(q, kc, vc, out, part, max_chunks, b, n_kv, cap, sp, stream);
-            default: return launch_gqa<T, 128, 8>(q, kc, vc, out, part, max_chunks, b, n_kv, cap, sp, stream);
+            case 1: return launch_gqa<T, 128, 1>(q, kc, vc, out, part, max_chunks, chunk, b, n_kv, cap, sp, stream);
+            case 2: return launch_gqa<T, 128, 2>(q, kc, vc, out, part, max_chunks, chunk, b, n_kv, cap, sp, stream);
+            case 4: return launch_gqa<T, 128, 4>(q, kc, vc, out, part, max_chunks, chunk, b, n_kv, cap, sp, stream);
+            default: return launch_gqa<T, 128, 8>(q, kc, vc, out, part, max_chunks, chunk, b, n_kv, cap, sp, stream);
         }
     }
     switch (gqa) {
-        case 1: return launch_gqa<T, 64, 1>(q, kc, vc, out, part, max_chunks, b, n_kv, cap, sp, stream);
-        case 2: return launch_gqa<T, 64, 2>(q, kc, vc, out, part, max_chunks, b, n_kv, cap, sp, stream);
-        case 4: return launch_gqa<T, 64, 4>(q, kc, vc, out, part, max_chunks, b, n_kv, cap, sp, stream);
-        default: return launch_gqa<T, 64, 8>(q, kc, vc, out, part, max_chunks, b, n_kv, cap, sp, stream);
+        case 1: return launch_gqa<T, 64, 1>(q, kc, vc, out, part, max_chunks, chunk, b, n_kv, cap, sp, stream);
+        case 2: return launch_gqa<T, 64, 2>(q, kc, vc, out, part, max_chunks, chunk, b, n_kv, cap, sp, stream);
+        case 4: return launch_gqa<T, 64, 4>(q, kc, vc, out, part, max_chunks, chunk, b, n_kv, cap, sp, stream);
+        default: return launch_gqa<T, 64, 8>(q, kc, vc, out, part, max_chunks, chunk, b, n_kv, cap, sp, stream);
     }
 }
 
-// Workspace bytes for splitting windows of up to max_window positions (0 when one chunk holds
-// them).
-inline size_t attn_workspace_bytes(int64_t b, int64_t n_kv, int64_t gqa, int64_t head_dim, int64_t max_window) {
-    if (b <= 0 || n_kv <= 0 || gqa <= 0 || head_dim <= 0 || max_window <= kChunk) return 0;
-    const int64_t chunks = (max_window + kChunk - 1) / kChunk;
+// Workspace bytes for splitting windows of up to max_window positions into chunks of `chunk` (0 when
+// one chunk holds them).
+inline size_t attn_workspace_bytes(int64_t b, int64_t n_kv, int64_t gqa, int64_t head_dim, int64_t max_window,
+                                   int chunk = kChunk) {
+    if (b <= 0 || n_kv <= 0 || gqa <= 0 || head_dim <= 0 || max_window <= chunk) return 0;
+    const int64_t chunks = (max_window + chunk - 1) / chunk;
     return static_cast<size_t>(b * n_kv * chunks * gqa * (head_dim + 2)) * sizeof(float);
 }
 

@@ -517,13 +517,14 @@ __global__ __launch_bounds__(256) void q8_merge(const float *part, float *y, int
 // does not fit it. W8A32 above 16 rows takes eight-block ranges: its two f16 slabs then leave room
 // for three workgroups per CU (52 KB at 48 rows, against 103 KB and one at sixteen blocks; the
 // gate|up projection at the talker's shape 41.6 -> 29.7 us), where the other modes measured
-// faster with the wider ranges.
+// faster with the wider ranges; up to 16 rows sixteen-block ranges at most (thirty-two hold 212
+// registers and 68 KB a workgroup: 8 rows, gate|up 21.6 -> 14.4 us, down 11.6 -> 9.7).
 int pick_q8_nb(int64_t m, int64_t k, int64_t n, int32_t mode) {
     const int64_t nblocks = k / 32, tiles = n / 64, rows = (m + 15) / 16 * 16;
     if (m <= 0 || m > 64 || n % 64 != 0 || nblocks % 8 != 0 || tiles >= 65536) return 0;
     if (mode == DTTS_Q8_W8A32 && m > 16) return 8;
     for (int nb : {32, 16})
-        if (nblocks % nb == 0 && tiles * (nblocks / nb) >= 192 && rows * (nb * 32 + 8) * 2 <= 65536) return nb;
+        if ((nb == 16 || mode != DTTS_Q8_W8A32) && nblocks % nb == 0 && tiles * (nblocks / nb) >= 192 && rows * (nb * 32 + 8) * 2 <= 65536) return nb;
     return 8;
 }
 

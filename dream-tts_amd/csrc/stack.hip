@@ -183,7 +183,7 @@ __global__ __launch_bounds__(256) void stack_gateup_merge(Partials gu, TO *t, in
 struct Plan {  // workspace carve-up for one (lanes, cap)
     size_t h, a16, t16, qkv, q, f32out, gemm_part, attn_part, total;
     size_t gemm_bytes, attn_bytes;
-    int max_window;
+    int max_window, attn_chunk;
 };
 
 Plan plan_of(const dtts_stack_geometry &g, int64_t lanes, int64_t cap) {
@@ -216,7 +216,8 @@ Plan plan_of(const dtts_stack_geometry &g, int64_t lanes, int64_t cap) {
     p.gemm_part = take(gb);
     const int64_t win = g.window > 0 && g.window < cap ? g.window : cap;
     p.max_window = static_cast<int>(win);
-    p.attn_bytes = attn_workspace_bytes(lanes, g.n_kv, g.heads / g.n_kv, g.head_dim, win);
+    p.attn_chunk = attn_step_chunk(lanes, g.n_kv, win);
+    p.attn_bytes = attn_workspace_bytes(lanes, g.n_kv, g.heads / g.n_kv, g.head_dim, win, p.attn_chunk);
     p.attn_part = take(p.attn_bytes);
     p.total = off;
     return p;
@@ -269,7 +270,6 @@ hipError_t enqueue_step(const dtts_stack &s, const float *x, float *out, const d
     float *q = reinterpret_cast<float *>(ws + pl.q);
     float *gpart = pl.gemm_bytes ? reinterpret_cast<float *>(ws + pl.gemm_part) : nullptr;
     float *apart = pl.attn_bytes ? reinterpret_cast<float *>(ws + pl.attn_part) : nullptr;
-    const int max_chunks = apart ? (pl.max_window + kChunk - 1) / kChunk : 0;
     const float qscale = g.qk_norm ? 1.0f : static_cast<float>(1.0 / std::sqrt(static_cast<double>(g.head_dim)));
     const DevSpans spans{s.pos, static_cast<int>(g.window)};
     // Projections the reference runs through candle's f16 matmul (lanes not a multiple of 8, or
@@ -296,7 +296,7 @@ hipError_t enqueue_step(const dtts_stack &s, const float *x, float *out, const d
             hd, cap, g.eps, qscale, r.ys, r.stride, r_qkv);
         STACK_STEP(hipGetLastError());
         STACK_STEP(launch_attention(q, reinterpret_cast<const half_t *>(caches[li].k),
-                                    reinterpret_cast<const half_t *>(caches[li].v), a16, apart, max_chunks, lanes,
+                                    reinterpret_cast<const half_t *>(caches[li].v), a16, apart, pl.max_window, pl.attn_chunk, lanes,
                                     n_kv, gqa, hd, cap, spans, stream));
         const float *attn_scale = g.layer_scale ? L.attn_scale : nullptr;
         if (r_o)
@@ -366,7 +366,7 @@ bool proj_shape_ok(int32_t how, int64_t k, int64_t n) {
 struct PlanW {  // workspace carve-up of the f32 / Q8_0 step
     size_t h, a, qkv, q, o, fbuf, t, part, attn_part, total;
     size_t part_bytes, attn_bytes;
-    int max_window;
+    int max_window, attn_chunk;
 };
 
 PlanW plan_w(const dtts_stack_geometry &g, int32_t how, int64_t lanes, int64_t cap) {
@@ -398,7 +398,8 @@ PlanW plan_w(const dtts_stack_geometry &g, int32_t how, int64_t lanes, int64_t c
     p.part = take(pb);
     const int64_t win = g.window > 0 && g.window < cap ? g.window : cap;
     p.max_window = static_cast<int>(win);
-    p.attn_bytes = attn_workspace_bytes(lanes, g.n_kv, g.heads / g.n_kv, g.head_dim, win);
+    p.attn_chunk = attn_step_chunk(lanes, g.n_kv, win);
+    p.attn_bytes = attn_workspace_bytes(lanes, g.n_kv, g.heads / g.n_kv, g.head_dim, win, p.attn_chunk);
     p.attn_part = take(p.attn_bytes);
     p.total = off;
     return p;
@@ -431,7 +432,6 @@ hipError_t enqueue_step_w(const dtts_stack &s, const float *x, float *out, const
     float *t = reinterpret_cast<float *>(ws + pl.t);
     float *part = pl.part_bytes ? reinterpret_cast<float *>(ws + pl.part) : nullptr;
     float *apart = pl.attn_bytes ? reinterpret_cast<float *>(ws + pl.attn_part) : nullptr;
-    const int max_chunks = apart ? (pl.max_window + kChunk - 1) / kChunk : 0;
     const float qscale = g.qk_norm ? 1.0f : static_cast<float>(1.0 / std::sqrt(static_cast<double>(g.head_dim)));
     const DevSpans spans{s.pos, static_cast<int>(g.window)};
     const int32_t how = s.how;
@@ -450,7 +450,7 @@ hipError_t enqueue_step_w(const dtts_stack &s, const float *x, float *out, const
             heads, n_kv, hd, cap, g.eps, qscale, r.ys, r.stride, false);
         STACK_STEP(hipGetLastError());
         STACK_STEP(launch_attention(q, static_cast<const float *>(kc), static_cast<const float *>(vc), o, apart,
-                                    max_chunks, lanes, n_kv, gqa, hd, cap, spans, stream));
+                                    pl.max_window, pl.attn_chunk, lanes, n_kv, gqa, hd, cap, spans, stream));
         const float *attn_scale = g.layer_scale ? L.attn_scale : nullptr;
         STACK_STEP(proj_w(how, o, L.wo, fbuf, part, lanes, qw, dim, r, stream));
         STACK_STEP(launch_norm(h, r, attn_scale, h, L.ffn_norm, a, lanes, dim, g.eps, stream));

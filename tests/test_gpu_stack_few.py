@@ -1,0 +1,53 @@
+"""The decode step at few lanes against the oracle, where its attention splits spans into shorter chunks:
+positions on both sides of a chunk's edge, one lane to the batch that fills the chip, both cache types,
+grouped heads and windows. Bars as test_gpu_stack.py's."""
+from dataclasses import replace
+
+import numpy as np
+import pytest
+import torch
+
+import oracle
+from dtts import stack, synth
+
+from _stack_ref import SMALL, WINDOWED, inputs
+from _util import rel, to_dev, to_host
+
+pytestmark = pytest.mark.gpu
+
+ONE = replace(SMALL, layers=1, capacity=1600)
+
+
+@pytest.mark.parametrize("geo,weight,lanes,cap,pos", [
+    (ONE, "f16", 1, 256, [255]),                      # one chunk
+    (ONE, "f16", 1, 257, [256]),                      # three chunks, the last of one position
+    (ONE, "f16", 3, 700, [0, 127, 128]),
+    (ONE, "f16", 8, 1600, [0, 1, 255, 256, 511, 512, 1023, 1599]),
+    (ONE, "f16", 50, 300, [(i * 37) % 300 for i in range(50)]),
+    (ONE, "q8_0_a32", 2, 1500, [1499, 128]),
+    (ONE, "f32", 9, 520, [0, 63, 64, 127, 128, 129, 384, 511, 519]),
+    (replace(ONE, n_kv=4), "f16", 2, 400, [399, 200]),  # one query head per kv head
+    (replace(ONE, heads=8, n_kv=1, head_dim=64), "f16", 2, 400, [399, 129]),  # eight
+    (replace(WINDOWED, layers=1, window=300, capacity=700), "f16", 4, 700, [10, 299, 300, 699]),
+])
+def test_step_few_lanes(dev, geo, weight, lanes, cap, pos):
+    layers, fn = stack.random_weights(geo, 11)
+    x, kc, vc = inputs(geo, 11, lanes, cap, weight=weight)
+    st = stack.Stack(geo, layers, fn, dev, weight)
+    state = st.new_state(lanes, cap)
+    put = to_dev if weight == "f16" else lambda a, d: torch.from_numpy(a).to(d)
+    state.k[0].copy_(put(kc[0], dev))
+    state.v[0].copy_(put(vc[0], dev))
+    pos = np.asarray(pos, np.int32)
+    want = oracle.stack_decode_f32(geo, layers, fn, x, kc, vc, pos, weight)
+    got = to_host(st.decode(to_dev(x, dev), state, pos))
+    torch.cuda.synchronize()
+    bar = 2e-4 if weight == "f16" else 1e-5
+    assert rel(got, want)[1] < bar, rel(got, want)
+    back = synth.from_f16_bits if weight == "f16" else np.asarray
+    for g, w in ((state.k[0], kc[0]), (state.v[0], vc[0])):
+        g = to_host(g) if weight == "f16" else g.cpu().numpy()
+        for i, p in enumerate(pos):
+            off = np.arange(cap) != p
+            assert np.array_equal(g[i][:, off], w[i][:, off])
+            assert rel(back(g[i][:, p]), back(w[i][:, p]))[1] < (1e-3 if weight == "f16" else 1e-5)
