@@ -41,7 +41,8 @@ int decode_attention(const char *name, const float *q, const T *kc, const T *vc,
         DTTS_REQUIRE(aligned(workspace, 16), "%s: misaligned workspace", name);
         part = static_cast<float *>(workspace);
     }
-    const hipError_t e = launch_attention(q, kc, vc, out, part, static_cast<int>(max_window), kChunk, b, n_kv, gqa, head_dim, cap, sp, stream);
+    const hipError_t e = launch_attention(q, const_cast<T *>(kc), const_cast<T *>(vc), out, part, static_cast<int>(max_window), kChunk,
+                                          b, n_kv, gqa, head_dim, cap, sp, NoStep{}, stream);  // the caches are only read
     DTTS_HIP_CHECK(e, name);
     return DTTS_OK;
 }

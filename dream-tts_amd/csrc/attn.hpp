@@ -25,8 +25,10 @@
 #pragma once
 
 #include <cmath>
+#include <type_traits>
 
 #include "common.hpp"
+#include "norm_rope.hpp"
 
 namespace dtts {
 namespace {
@@ -117,29 +119,93 @@ __device__ __forceinline__ float softmax_exp2(float x) { return __builtin_amdgcn
 // 28.8 -> 15.3 us a layer, the merge 4.8 -> 5.3.
 constexpr int kChunk = 512, kChunkMin = 128, kChunkFill = 768;
 
+constexpr int kStepFuseMax = 128;  // (lane, kv head) pairs up to which the step's attention makes its own q, k and v
+
 inline int attn_step_chunk(int64_t b, int64_t n_kv, int64_t max_window) {
     int c = kChunk;
     while (c > kChunkMin && b * n_kv * ((max_window + c - 1) / c) < kChunkFill) c /= 2;
     return c < 2 * kChunkMin && max_window <= 2 * kChunkMin ? 2 * kChunkMin : c;  // a short window stays whole
 }
 
-// Chunks of a lane's window [lo, hi) when split.
-__device__ __host__ inline int chunks_of(int lo, int hi, int chunk) { return (hi - lo + chunk - 1) / chunk; }
+// Chunks of a lane's window [lo, hi) when split; a chunk is a power of two.
+__device__ __host__ inline int chunks_of(int lo, int hi, int chunk) {
+    return (hi - lo + chunk - 1) >> (31 - __builtin_clz(static_cast<unsigned>(chunk)));
+}
+
+// The step's QK-norm, RoPE and cache append, done by the attention workgroups themselves (the same
+// arithmetic as qk_rope_kernel): each makes its kv head's queries from the QKV projection's output,
+// and the one whose chunk holds the new position also makes its k and v rows and writes the caches.
+// Every workgroup of a (lane, kv head) repeats the queries' 2 to 9 rows of D values, which come from
+// L2; the launch and its gap are gone. Where the launch does not fill the chip that is the faster way
+// (a predictor step at one lane 181 -> 169 us, 8 lanes of a Q8_0 talker 234 -> 227 for three layers);
+// at 48 lanes every workgroup's rows wait on it, 36 -> 48 us against the 5 us of qk_rope_kernel.
+struct QkvStep {
+    const float *qkv;      // [b, (heads + 2 n_kv) D], or ys partials of it `stride` floats apart
+    int ys;
+    int64_t stride;
+    bool round16;          // the summed output rounded to f16 first (candle's f16 matmul)
+    const float *norms;    // [q | k] weights, or null
+    const float *cos_t, *sin_t;
+    float eps, q_scale;    // q_scale: on the roped q of layers without QK-norm
+};
+struct NoStep {};
+
+// One row of D values by one wave: lane j holds dims j and j + D/2 (D = 64: lanes past 31 idle).
+// w: the norm weights, or null for v (no norm, no RoPE).
+template <int D>
+__device__ __forceinline__ void step_row(const QkvStep &s, const float *src, const float *w, bool rope, const float *cos_r,
+                                         const float *sin_r, int j, float &o1, float &o2) {
+#pragma clang fp contract(off)
+    constexpr int H = D / 2;
+    auto ld = [&](const float *p) {  // the first eight partials requested together, summed in order
+        float v8[8];
+#pragma unroll
+        for (int y = 0; y < 8; ++y)
+            if (y < s.ys) v8[y] = p[y * s.stride];
+        float v = v8[0];
+#pragma unroll
+        for (int y = 1; y < 8; ++y)
+            if (y < s.ys) v += v8[y];
+        for (int y = 8; y < s.ys; ++y) v += p[y * s.stride];
+        return s.round16 ? static_cast<float>(static_cast<half_t>(v)) : v;
+    };
+    float x1 = 0.0f, x2 = 0.0f;
+    if (j < H) {
+        x1 = ld(src + j);
+        x2 = ld(src + j + H);
+    }
+    o1 = x1;
+    o2 = x2;
+    if (!rope) return;
+    const float ss = wave_sum(x1 * x1 + x2 * x2);
+    if (w) {  // candle's rms_norm: (x / m) * w
+        const float m = sqrtf(ss / static_cast<float>(D) + s.eps);
+        if (j < H) {
+            x1 = (x1 / m) * w[j];
+            x2 = (x2 / m) * w[j + H];
+        }
+    }
+    if (j < H) rope_pair(x1, x2, cos_r[j], sin_r[j], o1, o2);
+}
 
 // T: cache element type; D: head dim (64 or 128); GQA: query heads per kv head; NW: waves;
 // Src: HostSpans or DevSpans; OutT: float, or half_t for a consumer that casts the result.
 // part == nullptr: blockIdx.y is 0 and the workgroup writes out. Otherwise blockIdx.y is a chunk
 // of `chunk` positions, and the workgroup writes its state to part (rows of D + 2 floats: the
 // weighted v sum, the weight sum, the max score) at [(bh * max_chunks + chunk) * GQA + g].
-template <typename T, int D, int GQA, int NW, typename Src, typename OutT>
-__global__ __launch_bounds__(NW * 64) void decode_attn_kernel(const float *q, const T *kc, const T *vc, OutT *out,
+// Step: QkvStep makes q and the new position here (q is unused; the caches are written at hi - 1), or
+// NoStep reads q.
+template <typename T, int D, int GQA, int NW, typename Src, typename OutT, typename Step>
+__global__ __launch_bounds__(NW * 64, (std::is_same<Step, QkvStep>::value && GQA <= 2 ? 4 : 1)) void decode_attn_kernel(const float *q, T *kc, T *vc, OutT *out,
                                                               float *part, int max_chunks, int chunk, int n_kv, int cap,
-                                                              Src sp) {
+                                                              Src sp, Step st) {
+    constexpr bool STEP = std::is_same<Step, QkvStep>::value;
     constexpr int E = D / 16;     // dimensions per lane
     constexpr int G = NW * 4;     // position groups
     constexpr int UNROLL = 4;     // positions whose rows are in flight per group
     __shared__ float sm_m[G][GQA], sm_l[G][GQA];
     __shared__ __attribute__((aligned(16))) float sm_acc[G][GQA][D];
+    float *sm_row = &sm_acc[0][0][0];  // STEP: the queries, k and v until the groups' states are written
     const int bh = blockIdx.x;  // lane * n_kv + kv head
     const int lane_idx = bh / n_kv;
     const int tid = threadIdx.x;
@@ -148,18 +214,57 @@ __global__ __launch_bounds__(NW * 64) void decode_attn_kernel(const float *q, co
     const int j = tid & 15;
     int lo, hi;
     sp.get(lane_idx, lo, hi);
+    if (part && static_cast<int>(blockIdx.y) >= chunks_of(lo, hi, chunk)) return;  // the whole workgroup
+    [[maybe_unused]] const int pos = hi - 1;  // the new position
     if (part) {
-        if (static_cast<int>(blockIdx.y) >= chunks_of(lo, hi, chunk)) return;  // the whole workgroup
         lo += blockIdx.y * chunk;
         hi = hi < lo + chunk ? hi : lo + chunk;
     }
-
+    [[maybe_unused]] const bool owns = STEP && hi == pos + 1;  // the chunk holds the new position
     float qv[GQA][E];
+    if constexpr (STEP) {
+        // the queries, then k and v of the new position, a row per wave in turn
+        const int kh = bh - lane_idx * n_kv;
+        const float *row = st.qkv + static_cast<int64_t>(lane_idx) * (GQA + 2) * n_kv * D;
+        const float *cos_r = st.cos_t + static_cast<int64_t>(pos) * (D / 2), *sin_r = st.sin_t + static_cast<int64_t>(pos) * (D / 2);
+        for (int task = wave; task < (owns ? GQA + 2 : GQA); task += NW) {
+            const int lane = tid & 63;
+            const bool is_q = task < GQA, is_v = task == GQA + 1;
+            const int h = is_q ? kh * GQA + task : (is_v ? GQA + 1 : GQA) * n_kv + kh;
+            float o1, o2;
+            step_row<D>(st, row + static_cast<int64_t>(h) * D, st.norms ? st.norms + (is_q ? 0 : D) : nullptr, !is_v, cos_r,
+                        sin_r, lane, o1, o2);
+            if (is_q && st.q_scale != 1.0f) {
+                o1 = o1 * st.q_scale;
+                o2 = o2 * st.q_scale;
+            }
+            if (lane < D / 2) {
+                if (!is_q) {  // as the cache holds them
+                    T *dst = (is_v ? vc : kc) + (static_cast<int64_t>(bh) * cap + pos) * D;
+                    const T c1 = static_cast<T>(o1), c2 = static_cast<T>(o2);
+                    dst[lane] = c1;
+                    dst[lane + D / 2] = c2;
+                    o1 = static_cast<float>(c1);
+                    o2 = static_cast<float>(c2);
+                }
+                float *r = sm_row + task * D;
+                r[lane] = o1;
+                r[lane + D / 2] = o2;
+            }
+        }
+        __syncthreads();
 #pragma unroll
-    for (int g = 0; g < GQA; ++g) {
-        const float *qp = q + (static_cast<int64_t>(bh) * GQA + g) * D + j * E;
+        for (int g = 0; g < GQA; ++g)
 #pragma unroll
-        for (int e = 0; e < E; ++e) qv[g][e] = qp[e] * kLog2e;
+            for (int e = 0; e < E; ++e) qv[g][e] = sm_row[g * D + j * E + e] * kLog2e;
+        if (owns) --hi;  // its row comes from LDS, below
+    } else {
+#pragma unroll
+        for (int g = 0; g < GQA; ++g) {
+            const float *qp = q + (static_cast<int64_t>(bh) * GQA + g) * D + j * E;
+#pragma unroll
+            for (int e = 0; e < E; ++e) qv[g][e] = qp[e] * kLog2e;
+        }
     }
     float m[GQA], l[GQA], acc[GQA][E];
 #pragma unroll
@@ -247,6 +352,18 @@ __global__ __launch_bounds__(NW * 64) void decode_attn_kernel(const float *q, co
         CacheRow<T>::load(vb + static_cast<int64_t>(p) * D, vr);
         step(kr, vr);
     }
+    if constexpr (STEP) {
+        if (owns && p == pos) {  // the group whose turn the new position is
+            float kr[E], vr[E];
+#pragma unroll
+            for (int e = 0; e < E; ++e) {
+                kr[e] = sm_row[GQA * D + j * E + e];
+                vr[e] = sm_row[(GQA + 1) * D + j * E + e];
+            }
+            step(kr, vr);
+        }
+        __syncthreads();  // the rows are read
+    }
 
     // combine the groups' states
 #pragma unroll
@@ -288,7 +405,8 @@ __global__ __launch_bounds__(NW * 64) void decode_attn_kernel(const float *q, co
 
 // Merges the chunk states of each (lane, kv head): out = sum_c num_c e^(m_c - M) / sum_c den_c
 // e^(m_c - M), M the largest m_c, chunks in order (m in log2 units, so 2^(m_c - M)).
-template <int D, int GQA, typename Src, typename OutT>
+// U: chunk states requested together (a loop would wait for each in turn).
+template <int D, int GQA, int U, typename Src, typename OutT>
 __global__ __launch_bounds__(256) void decode_attn_merge(const float *part, OutT *out, int max_chunks, int chunk,
                                                          int n_kv, Src sp) {
     const int bh = blockIdx.x;
@@ -296,7 +414,6 @@ __global__ __launch_bounds__(256) void decode_attn_merge(const float *part, OutT
     int lo, hi;
     sp.get(lane_idx, lo, hi);
     const int nch = chunks_of(lo, hi, chunk);
-    constexpr int U = 16;  // chunk states requested together (a loop would wait for each in turn)
     for (int t = threadIdx.x; t < GQA * D; t += 256) {
         const int g = t / D, d = t - (t / D) * D;
         const float *pr = part + (static_cast<int64_t>(bh) * max_chunks * GQA + g) * (D + 2);
@@ -345,43 +462,46 @@ constexpr size_t attn_lds_pad() {
     return stat < 160 * 1024 / wg ? (160 * 1024 / wg - stat) / 512 * 512 : 0;
 }
 
-template <typename T, int D, int GQA, typename Src, typename OutT>
-hipError_t launch_gqa(const float *q, const T *kc, const T *vc, OutT *out, float *part, int max_chunks, int chunk, int64_t b,
-                      int64_t n_kv, int64_t cap, const Src &sp, hipStream_t stream) {
+template <typename T, int D, int GQA, typename Src, typename OutT, typename Step>
+hipError_t launch_gqa(const float *q, T *kc, T *vc, OutT *out, float *part, int max_chunks, int chunk, int64_t b,
+                      int64_t n_kv, int64_t cap, const Src &sp, const Step &st, hipStream_t stream) {
     const unsigned grid = static_cast<unsigned>(b * n_kv);
     constexpr size_t pad = attn_lds_pad<T, D, GQA>();
     if (!part) {
-        decode_attn_kernel<T, D, GQA, 4, Src, OutT><<<grid, 256, pad, stream>>>(
-            q, kc, vc, out, nullptr, 0, 0, static_cast<int>(n_kv), static_cast<int>(cap), sp);
+        decode_attn_kernel<T, D, GQA, 4, Src, OutT, Step><<<grid, 256, pad, stream>>>(
+            q, kc, vc, out, nullptr, 0, 0, static_cast<int>(n_kv), static_cast<int>(cap), sp, st);
         return hipGetLastError();
     }
-    decode_attn_kernel<T, D, GQA, 4, Src, OutT><<<dim3(grid, max_chunks), 256, pad, stream>>>(
-        q, kc, vc, out, part, max_chunks, chunk, static_cast<int>(n_kv), static_cast<int>(cap), sp);
+    decode_attn_kernel<T, D, GQA, 4, Src, OutT, Step><<<dim3(grid, max_chunks), 256, pad, stream>>>(
+        q, kc, vc, out, part, max_chunks, chunk, static_cast<int>(n_kv), static_cast<int>(cap), sp, st);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    decode_attn_merge<D, GQA, Src, OutT><<<grid, 256, 0, stream>>>(part, out, max_chunks, chunk, static_cast<int>(n_kv), sp);
+    if (max_chunks <= 4)
+        decode_attn_merge<D, GQA, 4, Src, OutT><<<grid, 256, 0, stream>>>(part, out, max_chunks, chunk, static_cast<int>(n_kv), sp);
+    else
+        decode_attn_merge<D, GQA, 16, Src, OutT><<<grid, 256, 0, stream>>>(part, out, max_chunks, chunk, static_cast<int>(n_kv), sp);
     return hipGetLastError();
 }
 
 // gqa in {1, 2, 4, 8} and D in {64, 128}, checked by the caller.
-template <typename T, typename Src, typename OutT>
-hipError_t launch_attention(const float *q, const T *kc, const T *vc, OutT *out, float *part, int max_window,
+template <typename T, typename Src, typename OutT, typename Step>
+hipError_t launch_attention(const float *q, T *kc, T *vc, OutT *out, float *part, int max_window,
                             int chunk, int64_t b, int64_t n_kv, int64_t gqa, int64_t head_dim, int64_t cap, const Src &sp,
-                            hipStream_t stream) {
+                            const Step &st, hipStream_t stream) {
     const int max_chunks = part ? (max_window + chunk - 1) / chunk : 0;
     if (head_dim == 128) {
         switch (gqa) {
-            case 1: return launch_gqa<T, 128, 1>(q, kc, vc, out, part, max_chunks, chunk, b, n_kv, cap, sp, stream);
-            case 2: return launch_gqa<T, 128, 2>(q, kc, vc, out, part, max_chunks, chunk, b, n_kv, cap, sp, stream);
-            case 4: return launch_gqa<T, 128, 4>(q, kc, vc, out, part, max_chunks, chunk, b, n_kv, cap, sp, stream);
-            default: return launch_gqa<T, 128, 8>(q, kc, vc, out, part, max_chunks, chunk, b, n_kv, cap, sp, stream);
+            case 1: return launch_gqa<T, 128, 1>(q, kc, vc, out, part, max_chunks, chunk, b, n_kv, cap, sp, st, stream);
+            case 2: return launch_gqa<T, 128, 2>(q, kc, vc, out, part, max_chunks, chunk, b, n_kv, cap, sp, st, stream);
+            case 4: return launch_gqa<T, 128, 4>(q, kc, vc, out, part, max_chunks, chunk, b, n_kv, cap, sp, st, stream);
+            default: return launch_gqa<T, 128, 8>(q, kc, vc, out, part, max_chunks, chunk, b, n_kv, cap, sp, st, stream);
         }
     }
     switch (gqa) {
-        case 1: return launch_gqa<T, 64, 1>(q, kc, vc, out, part, max_chunks, chunk, b, n_kv, cap, sp, stream);
-        case 2: return launch_gqa<T, 64, 2>(q, kc, vc, out, part, max_chunks, chunk, b, n_kv, cap, sp, stream);
-        case 4: return launch_gqa<T, 64, 4>(q, kc, vc, out, part, max_chunks, chunk, b, n_kv, cap, sp, stream);
-        default: return launch_gqa<T, 64, 8>(q, kc, vc, out, part, max_chunks, chunk, b, n_kv, cap, sp, stream);
+        case 1: return launch_gqa<T, 64, 1>(q, kc, vc, out, part, max_chunks, chunk, b, n_kv, cap, sp, st, stream);
+        case 2: return launch_gqa<T, 64, 2>(q, kc, vc, out, part, max_chunks, chunk, b, n_kv, cap, sp, st, stream);
+        case 4: return launch_gqa<T, 64, 4>(q, kc, vc, out, part, max_chunks, chunk, b, n_kv, cap, sp, st, stream);
+        default: return launch_gqa<T, 64, 8>(q, kc, vc, out, part, max_chunks, chunk, b, n_kv, cap, sp, st, stream);
     }
 }
 

@@ -4,7 +4,7 @@
 //   h = x
 //   per layer:  a = f16(rms_norm(h, attn_norm))                      rms kernel
 //               qkv = a . Wqkv^T                    (f32)             NT GEMM
-//               q, cache[pos] <- QK-norm, RoPE, append (or RoPE, q*s)  qk-rope kernel
+//               q, cache[pos] <- QK-norm, RoPE, append (or RoPE, q*s);
 //               o = f16(attention(q, cache[window .. pos]))           decode attention
 //               h += (o . Wo^T) * attn_scale                          NT GEMM, residual epilogue
 //               a = f16(rms_norm(h, ffn_norm))                        rms kernel
@@ -255,6 +255,31 @@ bool skinny_eligible(int64_t m, int64_t k, int64_t n) { return m <= 48 && m % 8 
         if (e_ != hipSuccess) return e_;          \
     } while (0)
 
+// A layer's QK-norm, RoPE, cache append and attention from the QKV projection's output: one launch
+// (and the chunks' merge) where the (lane, kv head) pairs are few, else the qk-rope kernel first.
+template <typename T, typename OutT>
+hipError_t step_attention(const dtts_stack &s, const dtts_stack_layer &L, T *kc, T *vc, const Partials &qkv, bool round16,
+                          float *q, OutT *out, float *part, int max_window, int chunk, int lanes, int cap,
+                          hipStream_t stream) {
+    const dtts_stack_geometry &g = s.geo;
+    const int heads = static_cast<int>(g.heads), n_kv = static_cast<int>(g.n_kv), hd = static_cast<int>(g.head_dim);
+    const float *norms = g.qk_norm ? L.qk_norms : nullptr;
+    const float qscale = g.qk_norm ? 1.0f : static_cast<float>(1.0 / std::sqrt(static_cast<double>(g.head_dim)));
+    const DevSpans spans{s.pos, static_cast<int>(g.window)};
+    if (lanes * n_kv <= kStepFuseMax) {
+        const QkvStep st{qkv.p, qkv.ys, qkv.stride, round16, norms, s.cos_t, s.sin_t, g.eps, qscale};
+        return launch_attention(nullptr, kc, vc, out, part, max_window, chunk, lanes, n_kv, heads / n_kv, hd, cap, spans, st,
+                                stream);
+    }
+    const int waves = lanes * (heads + n_kv);
+    qk_rope_kernel<float, DevPositions, T><<<static_cast<unsigned>((waves + 3) / 4), 256, 0, stream>>>(
+        qkv.p, norms, s.cos_t, s.sin_t, DevPositions{s.pos}, q, nullptr, kc, vc, lanes, heads, n_kv, hd, cap, g.eps, qscale,
+        qkv.ys, qkv.stride, round16);
+    STACK_STEP(hipGetLastError());
+    return launch_attention(q, kc, vc, out, part, max_window, chunk, lanes, n_kv, heads / n_kv, hd, cap, spans, NoStep{},
+                            stream);
+}
+
 // Enqueues the step (after the positions are on the device).
 hipError_t enqueue_step(const dtts_stack &s, const float *x, float *out, const dtts_stack_cache *caches, int lanes,
                         int cap, char *ws, const Plan &pl, hipStream_t stream) {
@@ -262,7 +287,6 @@ hipError_t enqueue_step(const dtts_stack &s, const float *x, float *out, const d
     const int dim = static_cast<int>(g.dim), hd = static_cast<int>(g.head_dim);
     const int heads = static_cast<int>(g.heads), n_kv = static_cast<int>(g.n_kv), ffn = static_cast<int>(g.ffn);
     const int qw = heads * hd, qkvw = (heads + 2 * n_kv) * hd;
-    const int gqa = heads / n_kv;
     float *h = reinterpret_cast<float *>(ws + pl.h);
     half_t *a16 = reinterpret_cast<half_t *>(ws + pl.a16);
     half_t *t16 = reinterpret_cast<half_t *>(ws + pl.t16);
@@ -270,8 +294,6 @@ hipError_t enqueue_step(const dtts_stack &s, const float *x, float *out, const d
     float *q = reinterpret_cast<float *>(ws + pl.q);
     float *gpart = pl.gemm_bytes ? reinterpret_cast<float *>(ws + pl.gemm_part) : nullptr;
     float *apart = pl.attn_bytes ? reinterpret_cast<float *>(ws + pl.attn_part) : nullptr;
-    const float qscale = g.qk_norm ? 1.0f : static_cast<float>(1.0 / std::sqrt(static_cast<double>(g.head_dim)));
-    const DevSpans spans{s.pos, static_cast<int>(g.window)};
     // Projections the reference runs through candle's f16 matmul (lanes not a multiple of 8, or
     // more than 48: a single lane's decode among them) take the plain-output form here, and each
     // consumer rounds the summed output to f16 as that matmul's output is.
@@ -289,15 +311,9 @@ hipError_t enqueue_step(const dtts_stack &s, const float *x, float *out, const d
         Partials r{};
         STACK_STEP(stack_gemm<0>(a16, reinterpret_cast<const half_t *>(L.wqkv), qkv, nullptr, nullptr, lanes, dim, qkvw,
                                  gpart, qkv, r, stream));
-        const int waves = lanes * (heads + n_kv);
-        qk_rope_kernel<float, DevPositions><<<static_cast<unsigned>((waves + 3) / 4), 256, 0, stream>>>(
-            r.p, g.qk_norm ? L.qk_norms : nullptr, s.cos_t, s.sin_t, DevPositions{s.pos}, q, nullptr,
-            reinterpret_cast<half_t *>(caches[li].k), reinterpret_cast<half_t *>(caches[li].v), lanes, heads, n_kv,
-            hd, cap, g.eps, qscale, r.ys, r.stride, r_qkv);
-        STACK_STEP(hipGetLastError());
-        STACK_STEP(launch_attention(q, reinterpret_cast<const half_t *>(caches[li].k),
-                                    reinterpret_cast<const half_t *>(caches[li].v), a16, apart, pl.max_window, pl.attn_chunk, lanes,
-                                    n_kv, gqa, hd, cap, spans, stream));
+        STACK_STEP(step_attention(s, L, reinterpret_cast<half_t *>(caches[li].k),
+                                  reinterpret_cast<half_t *>(caches[li].v), r, r_qkv, q, a16, apart, pl.max_window,
+                                  pl.attn_chunk, lanes, cap, stream));
         const float *attn_scale = g.layer_scale ? L.attn_scale : nullptr;
         if (r_o)
             STACK_STEP(stack_gemm<0>(a16, reinterpret_cast<const half_t *>(L.wo), fbuf, nullptr, nullptr, lanes, qw, dim,
@@ -342,9 +358,8 @@ hipError_t enqueue_step(const dtts_stack &s, const float *x, float *out, const d
 // (crates/tts-nn/src/lib.rs:509-531): no f16 rounding anywhere in the step. Per layer:
 //   a = rms_norm(h)                          rms kernel (f32 out; adds the previous projection)
 //   qkv = proj(a)                            f32 (Proj::Dense) or Q8_0 (QMatMul) A-sharing kernel
-//   q, cache[pos] <- QK-norm, RoPE, append   qk-rope kernel on f32 caches (the composed route:
-//                                            rms_norm over each head, rope, slice_set in f32)
-//   o = attention(q, cache)                  decode attention over the f32 caches, f32 out
+//   q, cache[pos] <- QK-norm, RoPE, append   (the composed route: rms_norm over each head, rope,
+//   o = attention(q, cache)                  slice_set in f32) and decode attention, f32 out
 //   h += proj(o) * attn_scale                (summed by the next norm)
 //   t = swiglu_mul(proj_gate(a), proj_up(a)) gate|up rows in one projection, f32 merge
 //   h += proj(t) * mlp_scale
@@ -422,7 +437,6 @@ hipError_t enqueue_step_w(const dtts_stack &s, const float *x, float *out, const
     const int dim = static_cast<int>(g.dim), hd = static_cast<int>(g.head_dim);
     const int heads = static_cast<int>(g.heads), n_kv = static_cast<int>(g.n_kv), ffn = static_cast<int>(g.ffn);
     const int qw = heads * hd, qkvw = (heads + 2 * n_kv) * hd;
-    const int gqa = heads / n_kv;
     float *h = reinterpret_cast<float *>(ws + pl.h);
     float *a = reinterpret_cast<float *>(ws + pl.a);
     float *qkv = reinterpret_cast<float *>(ws + pl.qkv);
@@ -432,8 +446,6 @@ hipError_t enqueue_step_w(const dtts_stack &s, const float *x, float *out, const
     float *t = reinterpret_cast<float *>(ws + pl.t);
     float *part = pl.part_bytes ? reinterpret_cast<float *>(ws + pl.part) : nullptr;
     float *apart = pl.attn_bytes ? reinterpret_cast<float *>(ws + pl.attn_part) : nullptr;
-    const float qscale = g.qk_norm ? 1.0f : static_cast<float>(1.0 / std::sqrt(static_cast<double>(g.head_dim)));
-    const DevSpans spans{s.pos, static_cast<int>(g.window)};
     const int32_t how = s.how;
     Partials pending{};  // the previous layer's down projection, not yet in h
     const float *pending_scale = nullptr;
@@ -444,13 +456,8 @@ hipError_t enqueue_step_w(const dtts_stack &s, const float *x, float *out, const
         STACK_STEP(launch_norm(li == 0 ? x : h, pending, pending_scale, h, L.attn_norm, a, lanes, dim, g.eps, stream));
         Partials r{};
         STACK_STEP(proj_w(how, a, L.wqkv, qkv, part, lanes, dim, qkvw, r, stream));
-        const int waves = lanes * (heads + n_kv);
-        qk_rope_kernel<float, DevPositions, float><<<static_cast<unsigned>((waves + 3) / 4), 256, 0, stream>>>(
-            r.p, g.qk_norm ? L.qk_norms : nullptr, s.cos_t, s.sin_t, DevPositions{s.pos}, q, nullptr, kc, vc, lanes,
-            heads, n_kv, hd, cap, g.eps, qscale, r.ys, r.stride, false);
-        STACK_STEP(hipGetLastError());
-        STACK_STEP(launch_attention(q, static_cast<const float *>(kc), static_cast<const float *>(vc), o, apart,
-                                    pl.max_window, pl.attn_chunk, lanes, n_kv, gqa, hd, cap, spans, stream));
+        STACK_STEP(step_attention(s, L, kc, vc, r, false, q, o, apart, pl.max_window, pl.attn_chunk, lanes, cap,
+                                  stream));
         const float *attn_scale = g.layer_scale ? L.attn_scale : nullptr;
         STACK_STEP(proj_w(how, o, L.wo, fbuf, part, lanes, qw, dim, r, stream));
         STACK_STEP(launch_norm(h, r, attn_scale, h, L.ffn_norm, a, lanes, dim, g.eps, stream));
