@@ -293,5 +293,97 @@ __global__ __launch_bounds__(256) void qk_rope_span_kernel(const T *qkv, const f
     }
 }
 
+// The same for the stack's prefill, D in {64, 128} and every operand but norms 16-byte aligned: D/4
+// lanes per (row, head), a lane holding pairs 2j and 2j + 1, so that a wave covers 64 / (D/4) heads with
+// 8-byte f32 and 4-byte f16 accesses (one pair per lane moves half as much per instruction).
+// HBM-bound: 2 (or 4) bytes in and 4 to 6 out per value. 8 x 256 talker positions (59 MB):
+// 28.6 -> 20.7 us.
+template <int D, typename T>
+__global__ __launch_bounds__(256) void qk_rope_span_pairs(const T *qkv, const float *norms, const float *cos_t,
+                                                          const float *sin_t, float *q_out, float *kf, float *vf,
+                                                          half_t *kc, half_t *vc, int rows, int t, int start, int heads,
+                                                          int n_kv, int cap, float eps, int ys, int64_t ystride,
+                                                          bool round16) {
+#pragma clang fp contract(off)
+    typedef float float2_v __attribute__((ext_vector_type(2)));
+    typedef T T2 __attribute__((ext_vector_type(2)));
+    constexpr int H = D / 2, LPH = D / 4, HPW = 64 / LPH;
+    const int per = heads + n_kv;
+    const int64_t task = (static_cast<int64_t>(blockIdx.x) * 4 + (threadIdx.x >> 6)) * HPW + ((threadIdx.x & 63) / LPH);
+    const bool on = task < static_cast<int64_t>(rows) * per;  // every lane takes part in the reduction
+    const int row = on ? static_cast<int>(task / per) : 0, h = on ? static_cast<int>(task - static_cast<int64_t>(row) * per) : 0;
+    const int j = 2 * (threadIdx.x % LPH);  // pairs j and j + 1: dims j, j + 1 and their partners + H
+    const int bi = row / t, ti = row - bi * t, p = start + ti;
+    const T *src_row = qkv + static_cast<int64_t>(row) * (heads + 2 * n_kv) * D;
+    const bool is_q = h < heads;
+    auto ld = [&](const T *q) {  // the first eight ranges' partials requested together, summed in range order
+        T2 w[8];
+#pragma unroll
+        for (int y = 0; y < 8; ++y)
+            if (y < ys) w[y] = *reinterpret_cast<const T2 *>(q + y * ystride);
+        float2_v v = {static_cast<float>(w[0][0]), static_cast<float>(w[0][1])};
+#pragma unroll
+        for (int y = 1; y < 8; ++y)
+            if (y < ys) {
+                v[0] += static_cast<float>(w[y][0]);
+                v[1] += static_cast<float>(w[y][1]);
+            }
+        for (int y = 8; y < ys; ++y) {
+            const T2 u = *reinterpret_cast<const T2 *>(q + y * ystride);
+            v[0] += static_cast<float>(u[0]);
+            v[1] += static_cast<float>(u[1]);
+        }
+        if (round16)
+            v = float2_v{static_cast<float>(static_cast<half_t>(v[0])), static_cast<float>(static_cast<half_t>(v[1]))};
+        return v;
+    };
+    const int kh = h - heads;
+    float2_v x1 = ld(src_row + h * D + j), x2 = ld(src_row + h * D + H + j), v1 = {}, v2 = {};
+    if (!is_q) {
+        v1 = ld(src_row + (heads + n_kv + kh) * D + j);
+        v2 = ld(src_row + (heads + n_kv + kh) * D + H + j);
+    }
+    const float2_v c = *reinterpret_cast<const float2_v *>(cos_t + static_cast<int64_t>(p) * H + j);
+    const float2_v s = *reinterpret_cast<const float2_v *>(sin_t + static_cast<int64_t>(p) * H + j);
+    float ss = x1[0] * x1[0] + x1[1] * x1[1] + (x2[0] * x2[0] + x2[1] * x2[1]);
+#pragma unroll
+    for (int o = LPH / 2; o >= 1; o >>= 1) ss += __shfl_xor(ss, o, 64);
+    if (!on) return;
+    if (norms) {
+        const float m = sqrtf(ss / static_cast<float>(D) + eps);
+        const float *w = norms + (is_q ? 0 : D);
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+            x1[e] = (x1[e] / m) * w[j + e];
+            x2[e] = (x2[e] / m) * w[j + H + e];
+        }
+    }
+    float2_v o1, o2;
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+        float a, b;
+        rope_pair(x1[e], x2[e], c[e], s[e], a, b);
+        o1[e] = a;
+        o2[e] = b;
+    }
+    if (is_q) {
+        float *dq = q_out + ((static_cast<int64_t>(bi) * heads + h) * t + ti) * D + j;
+        *reinterpret_cast<float2_v *>(dq) = o1;
+        *reinterpret_cast<float2_v *>(dq + H) = o2;
+        return;
+    }
+    auto f16 = [](float2_v v) { return half2_t{static_cast<half_t>(v[0]), static_cast<half_t>(v[1])}; };
+    const int64_t dst = ((static_cast<int64_t>(bi) * n_kv + kh) * cap + p) * D + j;
+    const int64_t fdst = ((static_cast<int64_t>(bi) * n_kv + kh) * t + ti) * D + j;
+    *reinterpret_cast<half2_t *>(kc + dst) = f16(o1);
+    *reinterpret_cast<half2_t *>(kc + dst + H) = f16(o2);
+    *reinterpret_cast<half2_t *>(vc + dst) = f16(v1);
+    *reinterpret_cast<half2_t *>(vc + dst + H) = f16(v2);
+    *reinterpret_cast<float2_v *>(kf + fdst) = o1;
+    *reinterpret_cast<float2_v *>(kf + fdst + H) = o2;
+    *reinterpret_cast<float2_v *>(vf + fdst) = v1;
+    *reinterpret_cast<float2_v *>(vf + fdst + H) = v2;
+}
+
 }  // namespace
 }  // namespace dtts
