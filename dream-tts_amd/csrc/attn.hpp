@@ -505,13 +505,29 @@ hipError_t launch_attention(const float *q, T *kc, T *vc, OutT *out, float *part
     }
 }
 
-// Workspace bytes for splitting windows of up to max_window positions into chunks of `chunk` (0 when
+// Workspace bytes for splitting windows of up to max_window positions into chunks of kChunk (0 when
 // one chunk holds them).
-inline size_t attn_workspace_bytes(int64_t b, int64_t n_kv, int64_t gqa, int64_t head_dim, int64_t max_window,
-                                   int chunk = kChunk) {
-    if (b <= 0 || n_kv <= 0 || gqa <= 0 || head_dim <= 0 || max_window <= chunk) return 0;
-    const int64_t chunks = (max_window + chunk - 1) / chunk;
+inline size_t attn_workspace_bytes(int64_t b, int64_t n_kv, int64_t gqa, int64_t head_dim, int64_t max_window) {
+    if (b <= 0 || n_kv <= 0 || gqa <= 0 || head_dim <= 0 || max_window <= kChunk) return 0;
+    const int64_t chunks = (max_window + kChunk - 1) / kChunk;
     return static_cast<size_t>(b * n_kv * chunks * gqa * (head_dim + 2)) * sizeof(float);
+}
+
+// The stack step's workspace: room for every window up to max_window at any lane count up to b, so that
+// one sized for the largest batch and capacity serves the smaller ones, whose chunks are shorter (a chunk
+// below kChunk is taken only while twice its length gives under kChunkFill workgroups, so its chunks stay
+// under twice the filling count). From kChunkFill lanes on the need only grows with the lanes.
+inline size_t attn_step_workspace_bytes(int64_t b, int64_t n_kv, int64_t gqa, int64_t head_dim, int64_t max_window) {
+    if (b <= 0 || n_kv <= 0 || gqa <= 0 || head_dim <= 0 || max_window <= 2 * kChunkMin) return 0;
+    const int64_t shortest = (max_window + kChunkMin - 1) / kChunkMin, longest = (max_window + kChunk - 1) / kChunk;
+    int64_t rows = 0;
+    for (int64_t i = 1; i <= b && i <= kChunkFill; ++i) {
+        const int64_t l = i < kChunkFill ? i : b;
+        const int64_t fill = 2 * ((kChunkFill + l * n_kv - 1) / (l * n_kv));
+        const int64_t most = shortest < fill ? shortest : (fill > longest ? fill : longest);
+        rows = l * n_kv * most > rows ? l * n_kv * most : rows;
+    }
+    return static_cast<size_t>(rows * gqa * (head_dim + 2)) * sizeof(float);
 }
 
 }  // namespace

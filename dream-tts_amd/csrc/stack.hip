@@ -217,7 +217,7 @@ Plan plan_of(const dtts_stack_geometry &g, int64_t lanes, int64_t cap) {
     const int64_t win = g.window > 0 && g.window < cap ? g.window : cap;
     p.max_window = static_cast<int>(win);
     p.attn_chunk = attn_step_chunk(lanes, g.n_kv, win);
-    p.attn_bytes = attn_workspace_bytes(lanes, g.n_kv, g.heads / g.n_kv, g.head_dim, win, p.attn_chunk);
+    p.attn_bytes = attn_step_workspace_bytes(lanes, g.n_kv, g.heads / g.n_kv, g.head_dim, win);
     p.attn_part = take(p.attn_bytes);
     p.total = off;
     return p;
@@ -293,7 +293,7 @@ hipError_t enqueue_step(const dtts_stack &s, const float *x, float *out, const d
     float *qkv = reinterpret_cast<float *>(ws + pl.qkv);
     float *q = reinterpret_cast<float *>(ws + pl.q);
     float *gpart = pl.gemm_bytes ? reinterpret_cast<float *>(ws + pl.gemm_part) : nullptr;
-    float *apart = pl.attn_bytes ? reinterpret_cast<float *>(ws + pl.attn_part) : nullptr;
+    float *apart = pl.max_window > pl.attn_chunk ? reinterpret_cast<float *>(ws + pl.attn_part) : nullptr;
     // Projections the reference runs through candle's f16 matmul (lanes not a multiple of 8, or
     // more than 48: a single lane's decode among them) take the plain-output form here, and each
     // consumer rounds the summed output to f16 as that matmul's output is.
@@ -414,7 +414,7 @@ PlanW plan_w(const dtts_stack_geometry &g, int32_t how, int64_t lanes, int64_t c
     const int64_t win = g.window > 0 && g.window < cap ? g.window : cap;
     p.max_window = static_cast<int>(win);
     p.attn_chunk = attn_step_chunk(lanes, g.n_kv, win);
-    p.attn_bytes = attn_workspace_bytes(lanes, g.n_kv, g.heads / g.n_kv, g.head_dim, win, p.attn_chunk);
+    p.attn_bytes = attn_step_workspace_bytes(lanes, g.n_kv, g.heads / g.n_kv, g.head_dim, win);
     p.attn_part = take(p.attn_bytes);
     p.total = off;
     return p;
@@ -445,7 +445,7 @@ hipError_t enqueue_step_w(const dtts_stack &s, const float *x, float *out, const
     float *fbuf = reinterpret_cast<float *>(ws + pl.fbuf);
     float *t = reinterpret_cast<float *>(ws + pl.t);
     float *part = pl.part_bytes ? reinterpret_cast<float *>(ws + pl.part) : nullptr;
-    float *apart = pl.attn_bytes ? reinterpret_cast<float *>(ws + pl.attn_part) : nullptr;
+    float *apart = pl.max_window > pl.attn_chunk ? reinterpret_cast<float *>(ws + pl.attn_part) : nullptr;
     const int32_t how = s.how;
     Partials pending{};  // the previous layer's down projection, not yet in h
     const float *pending_scale = nullptr;

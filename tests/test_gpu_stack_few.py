@@ -51,3 +51,25 @@ def test_step_few_lanes(dev, geo, weight, lanes, cap, pos):
             off = np.arange(cap) != p
             assert np.array_equal(g[i][:, off], w[i][:, off])
             assert rel(back(g[i][:, p]), back(w[i][:, p]))[1] < (1e-3 if weight == "f16" else 1e-5)
+
+
+@pytest.mark.parametrize("weight", ["f16", "q8_0_a32", "f32"])
+@pytest.mark.parametrize("lanes,cap,few,short", [(48, 1600, 1, 1600), (48, 1600, 17, 700), (24, 600, 8, 257),
+                                                 (2, 512, 2, 300)])
+def test_workspace_of_the_largest_serves_the_smaller(dev, weight, lanes, cap, few, short):
+    layers, fn = stack.random_weights(ONE, 3)
+    st = stack.Stack(ONE, layers, fn, dev, weight)
+    assert all(st.workspace_bytes(n, c) <= st.workspace_bytes(n + 1, c) for n in range(1, lanes) for c in (short, cap))
+    assert st.workspace_bytes(few, short) <= st.workspace_bytes(lanes, cap)
+    state = st.new_state(few, short)
+    ws = torch.zeros(st.workspace_bytes(lanes, cap), dtype=torch.uint8, device=dev)
+    x, kc, vc = inputs(ONE, 3, few, short, weight=weight)
+    pos = np.asarray([(short - 1 - i * 37) % short for i in range(few)], np.int32)
+    want = oracle.stack_decode_f32(ONE, layers, fn, x, kc, vc, pos, weight)
+    x, kc, vc = inputs(ONE, 3, few, short, weight=weight)
+    put = to_dev if weight == "f16" else lambda a, d: torch.from_numpy(a).to(d)
+    state.k[0].copy_(put(kc[0], dev))
+    state.v[0].copy_(put(vc[0], dev))
+    got = to_host(st.decode(to_dev(x, dev), state, pos, workspace=ws))
+    torch.cuda.synchronize()
+    assert rel(got, want)[1] < (2e-4 if weight == "f16" else 1e-5)
