@@ -524,7 +524,9 @@ int pick_q8_nb(int64_t m, int64_t k, int64_t n, int32_t mode) {
     if (m <= 0 || m > 64 || n % 64 != 0 || nblocks % 8 != 0 || tiles >= 65536) return 0;
     if (mode == DTTS_Q8_W8A32 && m > 16) return 8;
     for (int nb : {32, 16})
-        if ((nb == 16 || mode != DTTS_Q8_W8A32) && nblocks % nb == 0 && tiles * (nblocks / nb) >= 192 && rows * (nb * 32 + 8) * 2 <= 65536) return nb;
+        if ((nb == 16 || mode != DTTS_Q8_W8A32) && nblocks % nb == 0 && tiles * (nblocks / nb) >= 192 &&
+            rows * (nb * 32 + 8) * 2 <= 65536)
+            return nb;
     return 8;
 }
 

@@ -271,19 +271,19 @@ __global__ __launch_bounds__(Cfg::THREADS, Cfg::WPE) void ru_nlc_f16(RuArgs q) {
                 w2r[i] = *reinterpret_cast<const half8_t *>(q.w2 + sg * 8);
         }
     };
-    w_issue(0, (smem + 0 * Cfg::STAGE));
+    w_issue(0, smem);
     win_load(R[0], 0);
     if (Cfg::CHUNKS > 1) win_load(R[1], KC);
     if (PD == 3 && Cfg::CHUNKS > 2) win_load(R[PD - 1], 2 * KC);
     wait_vmem_le<(Cfg::CHUNKS > PD - 1 ? PD - 1 : Cfg::CHUNKS - 1) * Cfg::A_PER_T>();  // W1 and chunk 0's window
-    win_store(R[0], 0, (smem + 0 * Cfg::STAGE));
+    win_store(R[0], 0, smem);
     stage_barrier();
-    if constexpr (KT > 0) load_frags((smem + 0 * Cfg::STAGE), 0, 0);
+    if constexpr (KT > 0) load_frags(smem, 0, 0);
 #pragma unroll
     for (int c = 0; c < Cfg::CHUNKS; ++c) {
         const int cur = c & 1, nxt = cur ^ 1;
         const bool last = c + 1 == Cfg::CHUNKS;
-        if (!last) w_issue((c + 1) * KC, (smem + nxt * Cfg::STAGE));
+        if (!last) w_issue((c + 1) * KC, smem + nxt * Cfg::STAGE);
         if (c + PD < Cfg::CHUNKS) win_load(R[c % PD], (c + PD) * KC);
         if (last) w2_load();
         const SnakeK kk = snake_consts((last ? c : c + 1) * KC);
@@ -308,13 +308,13 @@ __global__ __launch_bounds__(Cfg::THREADS, Cfg::WPE) void ru_nlc_f16(RuArgs q) {
 #pragma unroll
             for (int t = 0; t < KT; ++t) {
                 const int set = (c * KT + t) & 1;
-                if (t + 2 == KT && !last) win_write(Rn, (smem + nxt * Cfg::STAGE));
+                if (t + 2 == KT && !last) win_write(Rn, smem + nxt * Cfg::STAGE);
                 if (t + 1 < KT) {
-                    load_frags((smem + cur * Cfg::STAGE), t + 1, set ^ 1);
+                    load_frags(smem + cur * Cfg::STAGE, t + 1, set ^ 1);
                 } else {
                     wait_next();
                     stage_barrier();
-                    if (!last) load_frags((smem + nxt * Cfg::STAGE), 0, set ^ 1);
+                    if (!last) load_frags(smem + nxt * Cfg::STAGE, 0, set ^ 1);
                 }
                 mma(set);
                 if (t + 2 < KT && !last) snake_elems(Rn, kk, t * NE / (KT - 2), (t + 1) * NE / (KT - 2));
@@ -330,13 +330,13 @@ __global__ __launch_bounds__(Cfg::THREADS, Cfg::WPE) void ru_nlc_f16(RuArgs q) {
             }
         } else {
             for (int t = 0; t < k; ++t) {
-                load_frags((smem + cur * Cfg::STAGE), t, 0);
+                load_frags(smem + cur * Cfg::STAGE, t, 0);
                 mma(0);
             }
             if (!last) {
                 snake_elems(Rn, kk, 0, NE);
                 wait_next();
-                win_write(Rn, (smem + nxt * Cfg::STAGE));
+                win_write(Rn, smem + nxt * Cfg::STAGE);
             }
             stage_barrier();
         }
