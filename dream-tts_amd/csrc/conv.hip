@@ -209,12 +209,26 @@ Choice choose(const dtts_conv_desc *d) {
     return c;
 }
 
+// A k = 1 conv's positions are independent: the lanes as one sequence, so that a tile spans lanes
+// instead of padding each (10 x 325 rows: 26 tiles of 128 rows, 30 lane by lane).
+dtts_conv_desc as_one_sequence(const dtts_conv_desc &d) {
+    dtts_conv_desc f = d;
+    if (d.k == 1 && d.lanes > 1 && direct_offsets_fit(d.lanes * d.len, d.cin, d.cout, 1) &&
+        d.lanes * d.len * d.cout * 2 < (int64_t(1) << 31)) {
+        f.len = d.lanes * d.len;
+        f.lanes = 1;
+    }
+    return f;
+}
+
 }  // namespace
 
 const char *conv_path_name(const dtts_conv_desc *d) { return choose(d).path; }
 
-const char *conv_kernel_name(const dtts_conv_desc *d) {
+const char *conv_kernel_name(const dtts_conv_desc *desc) {
     static thread_local char buf[128];
+    const dtts_conv_desc seq = as_one_sequence(*desc);  // as it is launched
+    const dtts_conv_desc *d = &seq;
     const Choice c = choose(d);
     if (std::strcmp(c.path, "mfma") == 0)
         with_tile_k(c.kmax, d->lanes, static_cast<int>(d->len), static_cast<int>(d->cin), static_cast<int>(d->cout), c.direct_ok,
@@ -271,16 +285,9 @@ int conv1d_nlc_f16(const dtts_conv_desc *d, hipStream_t stream) {
     p.act = d->act;
     p.scale = d->out_scale;
 
-    // a k = 1 conv's positions are independent: the lanes as one sequence, so that a tile spans lanes
-    // instead of padding each (10 x 325 rows: 26 tiles of 128 rows, 30 lane by lane)
-    dtts_conv_desc flat = *d;
-    if (d->k == 1 && d->lanes > 1 && direct_offsets_fit(d->lanes * d->len, d->cin, d->cout, 1) &&
-        d->lanes * d->len * d->cout * 2 < (int64_t(1) << 31)) {
-        flat.len = d->lanes * d->len;
-        flat.lanes = 1;
-        p.L = static_cast<int>(flat.len);
-        d = &flat;
-    }
+    const dtts_conv_desc seq = as_one_sequence(*d);
+    p.L = static_cast<int>(seq.len);
+    d = &seq;
     const Choice ch = choose(d);
     hipError_t e;
     if (std::strcmp(ch.path, "narrow") == 0) {
