@@ -273,10 +273,15 @@ __global__ __launch_bounds__(256) void swiglu_rows_kernel(const half_t *gu, half
 //                           plus two shuffles (xor 16, 32). Scaled after the dot product, as the
 //                           prefill branch scales the scores; keys outside (q - window, q]
 //                           masked to -inf.
-//   p = exp(s - max)        rounded to f16 (the MFMA operand); sum over the rounded p in f32.
+//   p = 2^(s - max)         scores held in base 2; rounded to f16 (the MFMA operand); sum over the
+//                           rounded p in f32.
 //   out^T = V^T . P^T       two tiles of p per MFMA: a lane's own p values are the B operand as
 //                           they stand, with V^T's k slots permuted to the same keys (exact: the
-//                           sum over keys is order-free). out = acc / sum, one f16 rounding.
+//                           sum over keys is order-free). out = acc * (1 / sum), one f16 rounding.
+// Bound: instruction issue, four waves per SIMD of short f32 work around 24 MFMAs each. One v_exp_f32
+// per weight (the library expf takes ~12 instructions), one comparison per score for the mask and one
+// division per query: 10 x 325 x 16 heads, window 72: 17.3 -> 13.9 us. Requesting every staged row
+// and the query before the first use changed nothing (17.3).
 constexpr int kWinMax = 192;
 constexpr int kQBlock = 64;
 
@@ -349,6 +354,10 @@ __global__ __launch_bounds__(256) void window_attn_kernel(const half_t *qkv, con
     __syncthreads();
     if (l0 + 16 * w >= T) return;  // the whole wave is past the sequence (no barrier follows)
     // scores^T per tile: rows = keys 16 (w + t) + 4g + r of the staging, column = this query
+    // (in base 2). Key j = q - back is seen when 0 <= back < window and j >= 0, one unsigned comparison.
+    const float s2 = scale * 1.44269504088896341f;
+    const uint32_t seen = static_cast<uint32_t>(q < window ? q + 1 : window);
+    const int back0 = col + window - 1 - 4 * g;
     float s[NT][4];
     float mx = -INFINITY;
 #pragma unroll
@@ -361,9 +370,7 @@ __global__ __launch_bounds__(256) void window_attn_kernel(const half_t *qkv, con
         c = __builtin_amdgcn_mfma_f32_16x16x32_f16(kb, qb, c, 0, 0, 0);
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-            const int j = j0 + 16 * (w + t) + 4 * g + r;
-            const bool seen = j >= 0 && j <= q && j > q - window;
-            s[t][r] = seen ? c[r] * scale : -INFINITY;
+            s[t][r] = static_cast<uint32_t>(back0 - 16 * t - r) < seen ? c[r] * s2 : -INFINITY;
             mx = fmaxf(mx, s[t][r]);
         }
     }
@@ -376,7 +383,7 @@ __global__ __launch_bounds__(256) void window_attn_kernel(const half_t *qkv, con
     for (int t = 0; t < NT; ++t)
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-            p[t][r] = static_cast<half_t>(__builtin_expf(s[t][r] - mx));
+            p[t][r] = static_cast<half_t>(__builtin_amdgcn_exp2f(s[t][r] - mx));
             sum += static_cast<float>(p[t][r]);
         }
     sum += __shfl_xor(sum, 16, 64);
@@ -399,12 +406,13 @@ __global__ __launch_bounds__(256) void window_attn_kernel(const half_t *qkv, con
     }
     if (q >= T) return;
     // out^T tile dt: this lane holds dims 16 dt + 4g + r of its query
+    const float inv = 1.0f / sum;
     half_t *dst = out + (static_cast<int64_t>(lane_idx) * T + q) * heads * D + h * D + 4 * g;
 #pragma unroll
     for (int dt = 0; dt < 4; ++dt) {
         half4_t v;
 #pragma unroll
-        for (int r = 0; r < 4; ++r) v[r] = static_cast<half_t>(o[dt][r] / sum);
+        for (int r = 0; r < 4; ++r) v[r] = static_cast<half_t>(o[dt][r] * inv);
         *reinterpret_cast<half4_t *>(dst + 16 * dt) = v;
     }
 }
