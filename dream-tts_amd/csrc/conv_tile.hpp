@@ -807,7 +807,7 @@ __device__ __forceinline__ void conv_epilogue_form(const float16_t (&acc)[Cfg::T
                     break;
                 case 2:
 #pragma unroll
-                    for (int q = 0; q < 8; ++q) h[q] = static_cast<half_t>(conv_act(v[q], 2));
+                    for (int q = 0; q < 8; ++q) h[q] = f16_of_f32(conv_act(v[q], 2));
                     break;
                 case 3:
 #pragma unroll

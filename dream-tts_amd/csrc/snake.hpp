@@ -74,12 +74,22 @@ __device__ __forceinline__ void snake_f32_group(float (&v)[N], const float (&a)[
 // (crates/tts-nn/src/fused.rs:2356-2391).
 __device__ __forceinline__ float snake_f32(float x, float a, float r) { return x + r * sin2_f32(a, x); }
 
+// The f16 of an f32 value, which is rounded to f32 first in every kernel: the compiler turns a
+// product or fma and its conversion into v_fma_mixlo_f16 or v_fma_mixhi_f16 (one rounding) for some
+// elements of some instantiations and not for others, so that an element near an f16 midpoint took its
+// last bit from the tile it was computed on (a codec lane alone and in a batch differed). The empty asm
+// keeps the two apart; 12 x 10000 x 384, k = 7: 230.2 -> 231.2 us.
+__device__ __forceinline__ half_t f16_of_f32(float v) {
+    asm("" : "+v"(v));
+    return static_cast<half_t>(v);
+}
+
 // The f16-storage snake with ka = a / (2 pi) precomputed per channel: x * ka, fract, sin, s*s
 // and one fma (which reads x as f16 directly: v_fma_mix_f32) per element.
 __device__ __forceinline__ half_t snake_f16k(half_t x, float ka, float r) {
     const float xf = static_cast<float>(x);
     const float s = sin_rev_f16out(xf * ka);
-    return static_cast<half_t>(__builtin_fmaf(r, s * s, xf));
+    return f16_of_f32(__builtin_fmaf(r, s * s, xf));
 }
 
 // The same value from a and an f32 x that holds an f16 (every caller rounds x to f16 first). Fused

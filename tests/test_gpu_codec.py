@@ -66,6 +66,18 @@ def test_codec_lanes_are_independent(dev):
     assert np.array_equal(full[2:3], one)
 
 
+@pytest.mark.parametrize("dtype,lanes,frames", [("f16", 8, 25), ("f16", 24, 6), ("f32", 4, 25)])
+def test_codec_lane_alone_and_in_a_batch(dev, dtype, lanes, frames):
+    """The same bits from a lane alone, where the convs run on small tiles, and in a batch, at the
+    benchmark's geometry."""
+    geo = codec.CONFIG5
+    model = codec.Codec(geo, _weights(geo, 12), dev, dtype=dtype)
+    latent = torch.from_numpy(synth.normal(12, "latent", (lanes, frames, geo.latent_dim))).to(dev)
+    latent = latent.to(torch.float16 if dtype == "f16" else torch.float32)
+    full, one = model.decode(latent), model.decode(latent[3:4].contiguous())
+    assert torch.equal(full[3], one[0]), int((full[3] != one[0]).sum())
+
+
 def test_codec_profile_covers_every_launch(dev):
     geo = SMALL
     model = codec.Codec(geo, _weights(geo, 9), dev)

@@ -74,3 +74,23 @@ def test_small_tiles_epilogue_forms(dev, lanes, length, k, dil):
     _check(pre, _f64(x, w, b, k, dil) + x.double())
     p = pre.double()
     _check(y, p + act[1].double() * torch.sin(act[0].double() * p) ** 2)
+
+
+@pytest.mark.parametrize("lanes,length,cin,cout,k,dil", [
+    (24, 25, 1024, 1536, 7, 1), (48, 1000, 384, 384, 7, 1), (48, 800, 256, 512, 7, 1), (24, 25, 1536, 6144, 2, 1),
+    (24, 1000, 384, 768, 2, 1), (48, 200, 768, 768, 1, 1), (24, 1000, 384, 384, 1, 1),
+])
+def test_activation_forms_alone_and_in_a_batch(dev, lanes, length, cin, cout, k, dil):
+    """SnakeBeta, the residual and the activations round an output the same way on every tile of a class."""
+    x, w, b = _inputs(lanes, length, cin, cout, k, dev)
+    g = torch.Generator(device=dev)
+    g.manual_seed(cout)
+    act = (torch.rand(cout, generator=g, device=dev) + 0.5, torch.rand(cout, generator=g, device=dev) + 0.5)
+    res = torch.randn((lanes, length, cout), generator=g, device=dev).half()
+    scale = torch.rand(cout, generator=g, device=dev)
+    for form in (dict(snake_out=act), dict(residual=res, snake_out=act, want_pre=True), dict(act="gelu"),
+                 dict(residual=res, scale=scale)):
+        one = {key: v[3:4].contiguous() if key == "residual" else v for key, v in form.items()}
+        y, alone = nlc.conv1d(x, w, b, k=k, dilation=dil, **form), nlc.conv1d(x[3:4].contiguous(), w, b, k=k, dilation=dil, **one)
+        for a, c in zip(y, alone) if isinstance(y, tuple) else ((y, alone),):
+            assert torch.equal(a[3], c[0]), (list(form), int((a[3] != c[0]).sum()))
