@@ -702,8 +702,12 @@ __global__ __launch_bounds__(256) void prefill_attention(const float *q, const h
 // Bound: the f32 matrix rate, 2 D / 64 MFMAs of 64 cycles per wave and block, and the longest
 // workgroup of a causal block row (long rows are dispatched first). Talker prompts, per layer: 1 x 701
 // (352 workgroups) 166 us on prefill_attention -> 53, 8 x 256 (1024) 74 us with the scores in LDS -> 50.
-constexpr int kPrefillFlashMinT = 16;    // fewer queries leave most of a 32-query block idle
-constexpr int kPrefillFlashFill = 1024;  // workgroups past which two waves each fill the chip; four below
+constexpr int kPrefillFlashMinT = 16;  // fewer queries leave most of a 32-query block idle
+// Waves per workgroup, the same for every launch: the count is the order in which a query's keys are summed,
+// and a prompt's result does not depend on the prompts beside it. With two waves a one-layer talker prompt
+// is up to 20% slower below 1024 workgroups (2 x 448 after 300 positions: 220 -> 264 us) and within 2% from
+// there on, but for few long prompts (2 x 1000: 414 -> 443).
+constexpr int kPrefillFlashWaves = 4;
 
 template <int D, int NW>
 constexpr size_t prefill_flash_lds() {
@@ -896,13 +900,10 @@ template <int D>
 hipError_t launch_prefill_flash(const float *q, const half_t *kc, const half_t *vc, const float *kf, const float *vf,
                                 half_t *out, int lanes, int t, int start, int heads, int n_kv, int cap, int window,
                                 float scale, hipStream_t stream) {
+    constexpr int NW = kPrefillFlashWaves;
     const unsigned blocks = static_cast<unsigned>(lanes * ((t + 31) / 32) * heads);
-    if (blocks >= kPrefillFlashFill)
-        prefill_attention_flash<D, 2><<<blocks, 128, prefill_flash_lds<D, 2>(), stream>>>(q, kc, vc, kf, vf, out, t, start, heads,
-                                                                                        n_kv, cap, window, scale);
-    else
-        prefill_attention_flash<D, 4><<<blocks, 256, prefill_flash_lds<D, 4>(), stream>>>(q, kc, vc, kf, vf, out, t, start, heads,
-                                                                                        n_kv, cap, window, scale);
+    prefill_attention_flash<D, NW><<<blocks, 64 * NW, prefill_flash_lds<D, NW>(), stream>>>(q, kc, vc, kf, vf, out, t, start, heads,
+                                                                                          n_kv, cap, window, scale);
     return hipGetLastError();
 }
 

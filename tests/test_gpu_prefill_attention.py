@@ -1,7 +1,7 @@
 """The prefill's 32-query attention blocks at their edges, against the oracle with the prefill's bars
 (outputs 5e-4, written cache entries 1e-3): query counts around a block, key ranges that end inside a
 32-key block of either kind (the cache's rows, the new ones), windows that mask whole blocks for some
-of a block's queries, and both wave counts of the launch rule (two waves from 1024 workgroups on)."""
+of a block's queries, few and many workgroups."""
 from dataclasses import replace
 
 import pytest
@@ -38,3 +38,21 @@ def test_prefill_attention_blocks(dev, geo, lanes, t, start):
     assert rel(got, want)[1] < 5e-4, rel(got, want)
     for g, w in ((state.k[0], kc[0]), (state.v[0], vc[0])):
         assert rel(synth.from_f16_bits(to_host(g)), synth.from_f16_bits(w))[1] < 1e-3
+
+
+@pytest.mark.parametrize("geo,lanes,t,start", [(LONG, 40, 200, 5), (LONG, 3, 300, 40), (WIN, 70, 129, 0)])
+def test_prompt_alone_and_in_a_batch(dev, geo, lanes, t, start):
+    """A prompt of more than 128 positions gives the same bits alone and beside others, whether or not
+    the batch fills the chip."""
+    layers, fn = stack.random_weights(geo, 8)
+    _, kc, vc = inputs(geo, 8, lanes, start + t)
+    st = stack.Stack(geo, layers, fn, dev)
+    x = to_dev(synth.normal(8, "prefill.x", (lanes, t, geo.dim)), dev)
+    outs = []
+    for sl in (slice(0, lanes), slice(lanes - 1, lanes)):
+        state = st.new_state(sl.stop - sl.start, start + t)
+        state.k[0].copy_(to_dev(kc[0][sl], dev))
+        state.v[0].copy_(to_dev(vc[0][sl], dev))
+        outs.append((st.prefill(x[sl].contiguous(), state, start), state.k[0], state.v[0]))
+    for batch, alone in zip(*outs):
+        assert torch.equal(batch[-1], alone[0])
