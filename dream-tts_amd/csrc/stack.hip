@@ -711,7 +711,33 @@ constexpr int kPrefillFlashWaves = 4;
 
 template <int D, int NW>
 constexpr size_t prefill_flash_lds() {
-    return sizeof(float) * (NW * (D * 32 + 64) > 32 * (D + 4) ? NW * (D * 32 + 64) : 32 * (D + 4));
+    return sizeof(float) * (NW * (D * 32 + 65) > 32 * (D + 4) ? NW * (D * 32 + 65) : 32 * (D + 4));
+}
+
+// One query's attention over its own keys lo .. last alone, by one wave (D / 64 dimensions a lane).
+template <int D>
+__device__ void prefill_attention_visible(const float *q, const half_t *kc, const half_t *vc, const float *kf,
+                                          const float *vf, half_t *out, int start, int lo, int last, float s2) {
+    constexpr int PER = D / 64;
+    const int d0 = (threadIdx.x & 63) * PER;
+    float m = -INFINITY, l = 0.0f, o[PER] = {};
+    for (int j = lo; j <= last && l == l; ++j) {  // a NaN sum stays one
+        float dot = 0.0f, v[PER];
+#pragma unroll
+        for (int r = 0; r < PER; ++r) {
+            const int64_t at = static_cast<int64_t>(j < start ? j : j - start) * D + d0 + r;
+            dot += q[d0 + r] * (j < start ? static_cast<float>(kc[at]) : kf[at]);
+            v[r] = j < start ? static_cast<float>(vc[at]) : vf[at];
+        }
+        const float s = wave_sum(dot) * s2, mx = fmaxf(m, s), mu = mx == -INFINITY ? 0.0f : mx;
+        const float c = __builtin_amdgcn_exp2f(m - mu), p = __builtin_amdgcn_exp2f(s - mu);
+        m = mx;
+        l = l * c + p;
+#pragma unroll
+        for (int r = 0; r < PER; ++r) o[r] = o[r] * c + p * v[r];
+    }
+#pragma unroll
+    for (int r = 0; r < PER; ++r) out[d0 + r] = static_cast<half_t>(o[r] / l);
 }
 
 template <int D, int NW>
@@ -869,8 +895,8 @@ __global__ __launch_bounds__(64 * NW, 2) void prefill_attention_flash(const floa
         ms[w * 32 + l32] = m;
         ls[w * 32 + l32] = l;
     }
+    uint32_t *nans = reinterpret_cast<uint32_t *>(ls + NW * 32);  // per wave: the queries whose share has a NaN
     __syncthreads();
-    if (l32 >= nq) return;
     float mt = -INFINITY, den = 0.0f, f[NW];
 #pragma unroll
     for (int u = 0; u < NW; ++u) mt = fmaxf(mt, ms[u * 32 + l32]);
@@ -879,8 +905,10 @@ __global__ __launch_bounds__(64 * NW, 2) void prefill_attention_flash(const floa
         f[u] = __builtin_amdgcn_exp2f(ms[u * 32 + l32] - mt);  // 0 for a wave that saw no key of the query
         den += ls[u * 32 + l32] * f[u];
     }
-    half_t *dst = out + (static_cast<int64_t>(bi) * t + tq) * heads * D + h * D;
+    half_t *block = out + (static_cast<int64_t>(bi) * t + ti0) * heads * D + h * D;
+    half_t *dst = block + static_cast<int64_t>(l32) * heads * D;
     typedef half_t hv_t __attribute__((ext_vector_type(NDB)));
+    bool nan = false;
 #pragma unroll
     for (int i = 0; i < 16 / NW; ++i) {
         const int v = w * (16 / NW) + i;
@@ -890,10 +918,25 @@ __global__ __launch_bounds__(64 * NW, 2) void prefill_attention_flash(const floa
             float num = 0.0f;
 #pragma unroll
             for (int u = 0; u < NW; ++u) num += os[((u * NDB + db) * 16 + v) * 64 + lane] * f[u];
+            nan |= num != num;
             r[db] = static_cast<half_t>(num / den);
         }
-        *reinterpret_cast<hv_t *>(dst + NDB * (8 * (v >> 2) + 4 * hf + (v & 3))) = r;
+        if (l32 < nq) *reinterpret_cast<hv_t *>(dst + NDB * (8 * (v >> 2) + 4 * hf + (v & 3))) = r;
     }
+    // A value that is not finite times the weight 0 of a masked key is NaN: a query whose sum is NaN is done
+    // again over the keys it sees, so that such a value reaches only the queries it is visible to.
+    const uint64_t bad = __ballot(nan && l32 < nq);
+    if (lane == 0) nans[w] = static_cast<uint32_t>(bad | (bad >> 32));
+    __syncthreads();  // also: every share of the block's outputs is stored
+    uint32_t redo = 0;
+#pragma unroll
+    for (int u = 0; u < NW; ++u) redo |= nans[u];
+    const int64_t cache = (static_cast<int64_t>(bi) * n_kv + kh) * cap * D, fresh = (static_cast<int64_t>(bi) * n_kv + kh) * t * D;
+    for (int a = w; a < nq; a += NW)
+        if (redo >> a & 1)
+            prefill_attention_visible<D>(q + ((static_cast<int64_t>(bi) * heads + h) * t + ti0 + a) * D, kc + cache, vc + cache,
+                                         kf + fresh, vf + fresh, block + static_cast<int64_t>(a) * heads * D, start,
+                                         lo_of(ti0 + a), start + ti0 + a, s2);
 }
 
 template <int D>

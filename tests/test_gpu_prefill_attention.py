@@ -56,3 +56,51 @@ def test_prompt_alone_and_in_a_batch(dev, geo, lanes, t, start):
         outs.append((st.prefill(x[sl].contiguous(), state, start), state.k[0], state.v[0]))
     for batch, alone in zip(*outs):
         assert torch.equal(batch[-1], alone[0])
+
+
+@pytest.mark.parametrize("value", [float("nan"), float("inf")])
+@pytest.mark.parametrize("geo,lanes,t,start,at", [
+    (LONG, 1, 500, 0, 490), (LONG, 2, 100, 40, 33), (LONG, 1, 600, 300, 599), (LONG, 1, 20, 0, 19), (WIN, 1, 300, 500, 170),
+])
+def test_non_finite_position_stays_with_the_queries_that_see_it(dev, geo, lanes, t, start, at, value):
+    """A new position that is not finite leaves every earlier query's output as it is, and every query past
+    its window: its value is never multiplied into a query that does not see it."""
+    layers, fn = stack.random_weights(geo, 9)
+    _, kc, vc = inputs(geo, 9, lanes, start + t)
+    st = stack.Stack(geo, layers, fn, dev)
+    x = to_dev(synth.normal(9, "prefill.x", (lanes, t, geo.dim)), dev)
+
+    def run(x):
+        state = st.new_state(lanes, start + t)
+        state.k[0].copy_(to_dev(kc[0], dev))
+        state.v[0].copy_(to_dev(vc[0], dev))
+        return st.prefill(x, state, start)
+
+    want = run(x)
+    x[lanes - 1, at] = value
+    got = run(x)
+    seen = torch.zeros((lanes, t), dtype=torch.bool, device=dev)
+    seen[lanes - 1, at:min(t, at + geo.window) if geo.window else t] = True
+    assert torch.isfinite(got[~seen]).all()
+    assert rel(to_host(got[~seen]), to_host(want[~seen]))[1] < 5e-4
+    assert torch.isnan(got[seen]).all()
+
+
+def test_non_finite_cache_value_past_the_window(dev):
+    """An infinite cached value reaches the queries whose window holds it and no other of their block."""
+    layers, fn = stack.random_weights(WIN, 10)
+    t, start, at = 70, 90, 60  # seen by queries up to position 99, ti 9
+    _, kc, vc = inputs(WIN, 10, 1, start + t)
+    st = stack.Stack(WIN, layers, fn, dev)
+    x = to_dev(synth.normal(10, "prefill.x", (1, t, WIN.dim)), dev)
+    outs = []
+    for value in (None, float("inf")):
+        state = st.new_state(1, start + t)
+        state.k[0].copy_(to_dev(kc[0], dev))
+        state.v[0].copy_(to_dev(vc[0], dev))
+        if value:
+            state.v[0][0, :, at] = value
+        outs.append(st.prefill(x, state, start)[0])
+    seen = at + WIN.window - start
+    assert not torch.isfinite(outs[1][:seen]).any()
+    assert rel(to_host(outs[1][seen:]), to_host(outs[0][seen:]))[1] < 5e-4
