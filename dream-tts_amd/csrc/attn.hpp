@@ -119,8 +119,6 @@ __device__ __forceinline__ float softmax_exp2(float x) { return __builtin_amdgcn
 // 28.8 -> 15.3 us a layer, the merge 4.8 -> 5.3.
 constexpr int kChunk = 512, kChunkMin = 128, kChunkFill = 768;
 
-constexpr int kStepFuseMax = 128;  // (lane, kv head) pairs up to which the step's attention makes its own q, k and v
-
 inline int attn_step_chunk(int64_t b, int64_t n_kv, int64_t max_window) {
     int c = kChunk;
     while (c > kChunkMin && b * n_kv * ((max_window + c - 1) / c) < kChunkFill) c /= 2;
@@ -135,10 +133,16 @@ __device__ __host__ inline int chunks_of(int lo, int hi, int chunk) {
 // The step's QK-norm, RoPE and cache append, done by the attention workgroups themselves (the same
 // arithmetic as qk_rope_kernel): each makes its kv head's queries from the QKV projection's output,
 // and the one whose chunk holds the new position also makes its k and v rows and writes the caches.
-// Every workgroup of a (lane, kv head) repeats the queries' 2 to 9 rows of D values, which come from
-// L2; the launch and its gap are gone. Where the launch does not fill the chip that is the faster way
-// (a predictor step at one lane 181 -> 169 us, 8 lanes of a Q8_0 talker 234 -> 227 for three layers);
-// at 48 lanes every workgroup's rows wait on it, 36 -> 48 us against the 5 us of qk_rope_kernel.
+// Every chunk's workgroup repeats its GQA query rows of D values, which come from L2; the launch and its
+// gap are gone (a predictor step at one lane 181 -> 169 us). Up to kStepFuseMax (lane, kv head) pairs it
+// is the faster way at every window (two talker layers, f16 caches of 1536: 1 lane 111 -> 104.5 us, 16
+// lanes 140.3 -> 133.3), and beyond them while a window has at most two chunks (48 lanes: 257 positions
+// 142 -> 129 us, 800 6% to 12%, a predictor's 17 204 -> 191). With three chunks or more and more pairs it is
+// between 14% faster and 2% slower (48 lanes of 1536: 200.3 -> 202.0), and qk_rope_kernel stays.
+constexpr int kStepFuseMax = 128;
+
+inline bool step_fuses(int64_t pairs, int64_t chunks) { return pairs <= kStepFuseMax || chunks <= 2; }
+
 struct QkvStep {
     const float *qkv;      // [b, (heads + 2 n_kv) D], or ys partials of it `stride` floats apart
     int ys;

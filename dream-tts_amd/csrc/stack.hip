@@ -4,8 +4,8 @@
 //   h = x
 //   per layer:  a = f16(rms_norm(h, attn_norm))                      rms kernel
 //               qkv = a . Wqkv^T                    (f32)             NT GEMM
-//               q, cache[pos] <- QK-norm, RoPE, append (or RoPE, q*s);
-//               o = f16(attention(q, cache[window .. pos]))           decode attention
+//               q, cache[pos] <- QK-norm, RoPE, append (or RoPE, q*s)  decode attention, or the
+//               o = f16(attention(q, cache[window .. pos]))            qk-rope kernel and it
 //               h += (o . Wo^T) * attn_scale                          NT GEMM, residual epilogue
 //               a = f16(rms_norm(h, ffn_norm))                        rms kernel
 //               t = f16(silu(a . Wg^T) * (a . Wu^T))                  NT GEMM, gate|up epilogue
@@ -256,7 +256,7 @@ bool skinny_eligible(int64_t m, int64_t k, int64_t n) { return m <= 48 && m % 8 
     } while (0)
 
 // A layer's QK-norm, RoPE, cache append and attention from the QKV projection's output: one launch
-// (and the chunks' merge) where the (lane, kv head) pairs are few, else the qk-rope kernel first.
+// (and the chunks' merge) where step_fuses says so, else the qk-rope kernel first.
 template <typename T, typename OutT>
 hipError_t step_attention(const dtts_stack &s, const dtts_stack_layer &L, T *kc, T *vc, const Partials &qkv, bool round16,
                           float *q, OutT *out, float *part, int max_window, int chunk, int lanes, int cap,
@@ -266,7 +266,7 @@ hipError_t step_attention(const dtts_stack &s, const dtts_stack_layer &L, T *kc,
     const float *norms = g.qk_norm ? L.qk_norms : nullptr;
     const float qscale = g.qk_norm ? 1.0f : static_cast<float>(1.0 / std::sqrt(static_cast<double>(g.head_dim)));
     const DevSpans spans{s.pos, static_cast<int>(g.window)};
-    if (lanes * n_kv <= kStepFuseMax) {
+    if (step_fuses(lanes * n_kv, part ? (max_window + chunk - 1) / chunk : 1)) {
         const QkvStep st{qkv.p, qkv.ys, qkv.stride, round16, norms, s.cos_t, s.sin_t, g.eps, qscale};
         return launch_attention(nullptr, kc, vc, out, part, max_window, chunk, lanes, n_kv, heads / n_kv, hd, cap, spans, st,
                                 stream);

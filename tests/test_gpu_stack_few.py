@@ -1,6 +1,7 @@
 """The decode step at few lanes against the oracle, where its attention splits spans into shorter chunks:
 positions on both sides of a chunk's edge, one lane to the batch that fills the chip, both cache types,
-grouped heads and windows. Bars as test_gpu_stack.py's."""
+grouped heads and windows, on both sides of the line to which the attention makes its own q, k and v
+(128 (lane, kv head) pairs, or two chunks). Bars as test_gpu_stack.py's."""
 from dataclasses import replace
 
 import numpy as np
@@ -16,6 +17,14 @@ from _util import rel, to_dev, to_host
 pytestmark = pytest.mark.gpu
 
 ONE = replace(SMALL, layers=1, capacity=1600)
+EIGHT = replace(SMALL, layers=1, heads=8, n_kv=8, head_dim=64, capacity=1600)
+
+
+def edges(lanes, cap, chunk):
+    """A position per lane: both sides of every chunk's edge, the first and the last, in turn."""
+    at = sorted({p for e in range(0, cap + chunk, chunk) for p in (e - 1, e, e + 1) if 0 <= p < cap} | {cap - 1})
+    return [at[(i * 5) % len(at)] for i in range(lanes)]
+
 
 
 @pytest.mark.parametrize("geo,weight,lanes,cap,pos", [
@@ -29,6 +38,16 @@ ONE = replace(SMALL, layers=1, capacity=1600)
     (replace(ONE, n_kv=4), "f16", 2, 400, [399, 200]),  # one query head per kv head
     (replace(ONE, heads=8, n_kv=1, head_dim=64), "f16", 2, 400, [399, 129]),  # eight
     (replace(WINDOWED, layers=1, window=300, capacity=700), "f16", 4, 700, [10, 299, 300, 699]),
+    # more than 128 pairs: three chunks or more after the qk-rope kernel, up to two without it
+    (EIGHT, "f16", 17, 1100, edges(17, 1100, 128)), (EIGHT, "f32", 17, 1100, edges(17, 1100, 128)),
+    (EIGHT, "f16", 24, 1100, edges(24, 1100, 256)), (EIGHT, "f32", 33, 600, edges(33, 600, 256)),
+    (EIGHT, "f16", 48, 1536, edges(48, 1536, 512)), (EIGHT, "f32", 48, 1025, edges(48, 1025, 512)),
+    (replace(EIGHT, heads=16, head_dim=128), "f16", 24, 1100, edges(24, 1100, 256)),
+    (replace(WINDOWED, layers=1, heads=8, n_kv=8, window=700, capacity=1100), "f16", 24, 1100, edges(24, 1100, 256)),
+    (EIGHT, "f16", 48, 1000, edges(48, 1000, 512)), (EIGHT, "f32", 49, 257, edges(49, 257, 256)),
+    # (a multiple of 8 lanes: at 17 a projection's sum near a midpoint of its f16 rounding, 1.0959 against
+    # 1.0949, is one ulp of 2^-10 off, 2.7e-4 of the largest output, on either side of the line alike)
+    (replace(EIGHT, heads=16, head_dim=128), "f16", 24, 17, edges(24, 17, 16)),
 ])
 def test_step_few_lanes(dev, geo, weight, lanes, cap, pos):
     layers, fn = stack.random_weights(geo, 11)
