@@ -518,16 +518,23 @@ __global__ __launch_bounds__(256) void q8_merge(const float *part, float *y, int
 // for three workgroups per CU (52 KB at 48 rows, against 103 KB and one at sixteen blocks; the
 // gate|up projection at the talker's shape 41.6 -> 29.7 us), where the other modes measured
 // faster with the wider ranges; up to 16 rows sixteen-block ranges at most (thirty-two hold 212
-// registers and 68 KB a workgroup: 8 rows, gate|up 21.6 -> 14.4 us, down 11.6 -> 9.7).
-int pick_q8_nb(int64_t m, int64_t k, int64_t n, int32_t mode) {
+// registers and 68 KB a workgroup: 8 rows, gate|up 21.6 -> 14.4 us, down 11.6 -> 9.7), or the widest
+// again (`wide`) for a caller's workspace that holds no more ranges.
+int pick_q8_nb(int64_t m, int64_t k, int64_t n, int32_t mode, bool wide = false) {
     const int64_t nblocks = k / 32, tiles = n / 64, rows = (m + 15) / 16 * 16;
     if (m <= 0 || m > 64 || n % 64 != 0 || nblocks % 8 != 0 || tiles >= 65536) return 0;
     if (mode == DTTS_Q8_W8A32 && m > 16) return 8;
     for (int nb : {32, 16})
-        if ((nb == 16 || mode != DTTS_Q8_W8A32) && nblocks % nb == 0 && tiles * (nblocks / nb) >= 192 &&
+        if ((nb == 16 || wide || mode != DTTS_Q8_W8A32) && nblocks % nb == 0 && tiles * (nblocks / nb) >= 192 &&
             rows * (nb * 32 + 8) * 2 <= 65536)
             return nb;
     return 8;
+}
+
+// Bytes of the partial sums of k / 32 / nb ranges (one range writes y itself).
+size_t q8_range_bytes(int64_t m, int64_t k, int64_t n, int nb) {
+    const int64_t ranges = nb ? k / 32 / nb : 1;
+    return ranges > 1 ? static_cast<size_t>(ranges * m * n) * sizeof(float) : 0;
 }
 
 // GGML blocks -> the packed layout: row n is k bytes of quantised weights, lane-group major
@@ -833,8 +840,10 @@ int q8_packed(const char *name, const XT *x, const void *packed, float *y, int64
         DTTS_REQUIRE(aligned(x, 16) && aligned(packed, 16), "%s: x and packed must be 16-byte aligned", name);
         return q8_row_launch(name, x, packed, y, m, k, n, nbw, true, stream);
     }
-    const int nb = pick_q8_nb(m, k, n, mode);
-    const size_t need = dtts_gemm_q8_0_workspace_bytes(m, k, n);
+    // the narrower W8A32 ranges where the workspace holds them; the wider ones are enough to be taken
+    int nb = pick_q8_nb(m, k, n, mode);
+    if (q8_range_bytes(m, k, n, nb) > (workspace ? ws_bytes : 0)) nb = pick_q8_nb(m, k, n, mode, true);
+    const size_t need = q8_range_bytes(m, k, n, pick_q8_nb(m, k, n, DTTS_Q8_W8A32, true));
     DTTS_REQUIRE(nb > 0, "%s: shape not supported", name);
     DTTS_REQUIRE(!need || (workspace && ws_bytes >= need), "%s: workspace %zu bytes < %zu needed", name, ws_bytes, need);
     DTTS_REQUIRE(aligned(x, 16) && aligned(packed, 16) && (!need || aligned(workspace, 16)),
@@ -873,9 +882,7 @@ extern "C" int dtts_gemm_q8_0_f32(const float *x, const void *blocks, float *y, 
 
 extern "C" size_t dtts_gemm_q8_0_workspace_bytes(int64_t m, int64_t k, int64_t n) {
     if (m <= 0 || k <= 0 || n <= 0 || k % 32 != 0) return 0;
-    const int nb = dtts::pick_q8_nb(m, k, n, DTTS_Q8_W8A32);  // the mode with the most ranges
-    const int64_t ranges = nb ? k / 32 / nb : 1;
-    return ranges > 1 ? static_cast<size_t>(ranges * m * n) * sizeof(float) : 0;
+    return dtts::q8_range_bytes(m, k, n, dtts::pick_q8_nb(m, k, n, DTTS_Q8_W8A32));  // the mode with the most ranges
 }
 
 extern "C" int dtts_gemm_q8_0_ws(const dtts_f16 *x, const void *blocks, float *y, int64_t m, int64_t k, int64_t n,

@@ -13,7 +13,7 @@ import pytest
 import torch
 
 import oracle
-from dtts import ops, synth
+from dtts import DttsError, ops, synth
 
 from _util import rel, to_dev, to_host
 
@@ -167,6 +167,30 @@ def test_q8_0_packed_layout(dev, m, k, n):
     if m > 16:
         for mode, got in (("w8a8", got8), ("w8a16", got16)):
             assert np.array_equal(got, to_host(ops.q8_0_matmul(xd, bd, mode, workspace="auto"))), mode
+
+
+@pytest.mark.parametrize("k,n,ranges", [(1024, 12288, 1), (2048, 6400, 2), (2048, 12288, 2), (1024, 64, 4)])
+def test_q8_0_packed_takes_the_widest_ranges_workspace(dev, k, n, ranges):
+    """Up to 16 rows a workspace for the widest k ranges (none at all for one range) is enough in every
+    mode; W8A32 takes more, shorter ranges where the workspace holds them, with the same bars."""
+    m = 8
+    w = synth.normal(86, "w", (n, k), 0, 0.02)
+    blocks = ops.q8_0_quantize(w)
+    packed = ops.q8_0_repack(torch.from_numpy(blocks).to(dev), k)
+    x = synth.normal(86, "x", (m, k)).astype(np.float32)
+    need = ranges * m * n * 4 if ranges > 1 else 0
+    ws = torch.empty(need, dtype=torch.uint8, device=dev)
+    for mode in ("w8a32", "w8a8"):
+        xd = to_dev(x, dev)
+        got = to_host(ops.q8_0_matmul_packed(xd, packed, n, mode, workspace=ws))
+        want = oracle.q8_0_matmul_f64(x, blocks) if mode == "w8a32" else oracle.q8_0_matmul_w8a8(x, blocks)
+        assert rel(got, want)[1] <= 1e-5, mode
+        assert rel(to_host(ops.q8_0_matmul_packed(xd, packed, n, mode)), want)[1] <= 1e-5, mode
+    xh = to_dev(synth.f16_bits(x), dev)
+    assert torch.equal(ops.q8_0_matmul_packed(xh, packed, n, "w8a16", workspace=ws), ops.q8_0_matmul_packed(xh, packed, n, "w8a16"))
+    if need:
+        with pytest.raises(DttsError, match="workspace"):
+            ops.q8_0_matmul_packed(to_dev(x, dev), packed, n, "w8a8", workspace=ws[: need - 1])
 
 
 # ---------------------------------------------------------------- Q8_0 on f32 activations
