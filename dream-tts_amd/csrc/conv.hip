@@ -109,9 +109,15 @@ template <int KMAX, int HMAX, typename F>
 auto with_tile(int64_t lanes, int len, int cin, int cout, bool direct, F &&f) {
     if (direct) {
         // k <= 7 (dilated), 32-channel steps: eight waves of 64 x 96 or 32 x 96, or four of 32 x BN when those leave
-        // most CUs without a tile (three or four stages then: a lone tile waits on its loads)
+        // most CUs without a tile (three or four stages then: a lone tile waits on its loads). At widths that
+        // are no multiple of 96 the direct tiles are four waves of one 32 x 64 or 32 x 32 block each, half the
+        // register-staged tile's MFMAs per fragment read: they win while that one gives fewer than 160
+        // workgroups (1 x 3000 x 256 -> 512, k = 7, 96 of them: 10.9 us, 18.0 register-staged), it from there on
+        // (1 x 6000: 21.0 and 19.2; 16 x 3000: 127 and 103; 48 x 1500 x 64 -> 160, k = 3: 36 and 16).
         if constexpr (KMAX == 7) {
-            switch (pick_tile(kTile7, kTile7Count, lanes, len, cout)) {
+            const int64_t staged = lanes * ((len + 255) / 256) * (cout / (cout % 64 == 0 ? 64 : 32));
+            const int pick = cout % 96 != 0 && staged >= 160 ? -1 : pick_tile(kTile7, kTile7Count, lanes, len, cout);
+            switch (pick) {
                 case kTile7_512x96: return f(Tile<ConvTile<512, 96, 8, 1, 32, KMAX, HMAX, 2, kStageDirect>>{});
                 case kTile7_256x96: return f(Tile<ConvTile<256, 96, 8, 1, 32, KMAX, HMAX, 2, kStageDirect>>{});
                 case kTile7_128x96: return f(Tile<ConvTile<128, 96, 4, 1, 32, KMAX, HMAX, 2, kStageDirect>>{});

@@ -1,0 +1,43 @@
+"""Which tile a conv runs on, by the library's own kernel-name functions (no GPU): the lines at which the
+tap classes change tiles, on both sides. The tiles themselves are held to float64 and to each other's
+bits in test_gpu_conv_tiles.py."""
+import ctypes
+import re
+
+import pytest
+
+from dtts import lib
+from dtts.nlc import ConvDesc
+
+
+def tile(lanes, length, cin, cout, k, dil=1):
+    """(BM, BN, KC, stages, direct staging) of an f16 conv."""
+    fn = getattr(lib(), "_ZN4dtts16conv_kernel_nameEPK14dtts_conv_desc")
+    fn.restype = ctypes.c_char_p
+    d = ConvDesc(lanes, length, cin, cout, k, dil, (k - 1) * dil)
+    return _tile(fn(ctypes.byref(d)).decode())
+
+
+def split_tile(lanes, length, cin, cout, k, dil=1):
+    """The same of an f32 conv on the split route."""
+    fn = getattr(lib(), "_ZN4dtts22conv_split_kernel_nameEllllll")
+    fn.restype, fn.argtypes = ctypes.c_char_p, [ctypes.c_int64] * 6
+    return _tile(fn(lanes, length, cin, cout, k, dil).decode())
+
+
+def _tile(name):
+    bm, bn, _, _, kc, _, _, stages, staging = map(int, re.search(r"ConvTile<([^>]*)>", name).group(1).split(", "))
+    return bm, bn, kc, stages, staging == 1
+
+
+@pytest.mark.parametrize("lanes,length,cin,cout,k,want", [
+    # up to 159 register-staged workgroups of 256 x 64 (or 32): the small direct tiles
+    (1, 3000, 256, 512, 7, (128, 64)), (1, 50, 256, 512, 3, (128, 32)), (159, 200, 64, 64, 7, (128, 64)),
+    (159, 200, 64, 32, 5, (128, 32)),
+    # from 160 on: register-staged
+    (160, 200, 64, 64, 7, (256, 64)), (1, 6000, 256, 512, 7, (256, 64)), (48, 1500, 64, 160, 3, (256, 32)),
+    (16, 3000, 256, 512, 7, (256, 64)), (48, 1500, 32, 32, 3, (256, 32)),
+])
+def test_narrow_widths_up_to_seven_taps(lanes, length, cin, cout, k, want):
+    got = tile(lanes, length, cin, cout, k)
+    assert got[:2] == want and got[4] == (want[0] == 128)
