@@ -111,22 +111,29 @@ inline int pick_tiles_ng(int tiles_n, int64_t slice_bytes, int64_t budget = int6
     return best;
 }
 
-// Which tile a direct-staging conv runs on. A launch of r = tiles / 256 workgroups per CU is
-// estimated at full * floor(r), plus `light` for a last, partly filled round (a tile whose CU and
-// power budget it does not share takes `light`); the tile with the smallest estimate wins. The
-// costs are microseconds per KC-sized step of the reduction, measured over the codec's, the front
-// half's and the decoder stack's shapes at 1 to 48 lanes; the common factor, the step count,
-// is left out.
+// Which tile a direct-staging conv runs on: the one with the smallest estimated launch time. A round of
+// 256 workgroups (one per CU) takes `full`, a last, partly filled round `light` (its CUs and power budget
+// are shared with few others), and one of more than kLightTiles after full ones in proportion up to `full`:
+// 504 tiles of 256 x 96 are two rounds (4 x 16000 x 192, k = 7: 38.4 us, 35.2 on 256 tiles of 512 x 96).
+// A lone round stays `light`: the codec decodes its lanes as two halves side by side, and one's launches
+// run on the CUs that the other's leave. The costs are microseconds per KC-sized step of the reduction,
+// from single shapes launched repeatedly (operands warm: inside a prefill the same launches take 1.25 to
+// 1.5 times as long); the common factor, the step count, is left out.
 struct TileCost {
     int bm, bn;
     double full, light;
 };
 
+constexpr int kLightTiles = 192;
+
 inline double tile_cost(const TileCost &t, int64_t lanes, int64_t len, int64_t cout) {
     const int64_t tiles = lanes * ((len + t.bm - 1) / t.bm) * (cout / t.bn);
     const int64_t whole = tiles / 256, part = tiles % 256;
     if (whole == 0 || tiles == 256) return whole && t.full > t.light ? t.full : t.light;
-    return static_cast<double>(whole) * t.full + (part ? t.light : 0.0);
+    double last = part ? t.light : 0.0;
+    if (part > kLightTiles && t.full > t.light)
+        last += (t.full - t.light) * static_cast<double>(part - kLightTiles) / (256 - kLightTiles);
+    return static_cast<double>(whole) * t.full + last;
 }
 
 // The cheapest of n tiles whose bn divides cout (-1: none does).

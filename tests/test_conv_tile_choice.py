@@ -41,3 +41,13 @@ def _tile(name):
 def test_narrow_widths_up_to_seven_taps(lanes, length, cin, cout, k, want):
     got = tile(lanes, length, cin, cout, k)
     assert got[:2] == want and got[4] == (want[0] == 128)
+
+
+@pytest.mark.parametrize("lanes,length,channels,want", [
+    (4, 16000, 192, (512, 96)), (1, 16000, 768, (512, 96)),  # one full round, or two of half the tile
+    (24, 2000, 768, (512, 96)), (12, 10000, 384, (512, 96)), (4, 2000, 768, (256, 96)), (1, 1000, 384, (128, 32)),
+    (1, 200, 768, (128, 32)), (8, 500, 384, (128, 64)),
+])
+def test_seven_taps(lanes, length, channels, want):
+    assert tile(lanes, length, channels, channels, 7, 3)[:2] == want
+    assert split_tile(lanes, length, channels, channels, 7, 3)[:2] == want
