@@ -134,9 +134,8 @@ auto with_tile(int64_t lanes, int len, int cin, int cout, bool direct, F &&f) {
         // 32-channel stages: the smaller footprint (more workgroups per CU) beats a third stage in
         // flight, 9% at 128 x 128 and 16% at 128 x 96 on the codec's shapes.
         if constexpr (KMAX == 2) {
-            const int64_t tiles128 = lanes * ((len + 127) / 128) * (cout / 128);
             const int64_t tiles256 = lanes * ((len + 255) / 256) * (cout / 128);
-            if (cout % 64 == 0 && tiles128 < 192)
+            if (cout % 64 == 0 && few_tiles_k2(lanes, len, cout))
                 return f(Tile<ConvTile<64, 64, 2, 2, 32, KMAX, HMAX, 4, kStageDirect>>{});
             if (cout % 128 == 0 && cin >= 768 && tiles256 >= 224)
                 return f(Tile<ConvTile<256, 128, 2, 2, 32, KMAX, HMAX, 2, kStageDirect>>{});

@@ -194,9 +194,8 @@ bool with_split_tile(int64_t lanes, int len, int cin, int cout, F &&f) {
         }
     }
     if constexpr (KMAX == 2) {
-        const int64_t tiles128 = lanes * ((len + 127) / 128) * (cout / 128);
         const int64_t tiles256 = lanes * ((len + 255) / 256) * (cout / 128);
-        if ((cout % 128 == 0 || cout % 96 == 0) && cout % 64 == 0 && tiles128 < 192)
+        if ((cout % 128 == 0 || cout % 96 == 0) && cout % 64 == 0 && few_tiles_k2(lanes, len, cout))
             return f(STile<ConvTile<64, 64, 2, 2, 32, KMAX, HMAX, 4, kStageDirect>>{}), true;
         if (cout % 128 == 0 && cin >= 768 && tiles256 >= 224)
             return f(STile<ConvTile<256, 128, 2, 2, 32, KMAX, HMAX, 2, kStageDirect>>{}), true;

@@ -155,6 +155,15 @@ enum { kTile7_512x96, kTile7_256x96, kTile7_128x96, kTile7_128x64, kTile7_128x32
 constexpr TileCost kTile7[kTile7Count] = {
     {512, 96, 4.70, 2.70}, {256, 96, 2.62, 1.60}, {128, 96, 1.63, 1.14}, {128, 64, 1.10, 0.86}, {128, 32, 0.71, 0.67}};
 
+// Whether a k = 2 conv's positions and channels are few enough for 64 x 64 tiles, counted in 128 x 128 ones:
+// under 192, or 128 at 96-multiples, which otherwise run on 128 x 96. 1 x 9000 x 768 -> 192 (106): 13.9 us, 16.5 on
+// 128 x 96; 1 x 12000 (141): 20.2 and 16.7; 1 x 9000 x 384 -> 320 (177): 12.6, 13.7 register-staged; 1 x 12000
+// (235): 16.1 and 14.3; 48 x 5000 x 512 -> 64 (960): 75 and 61.
+inline bool few_tiles_k2(int64_t lanes, int64_t len, int64_t cout) {
+    const int64_t limit = cout % 128 != 0 && cout % 96 == 0 ? 128 : 192;
+    return lanes * ((len + 127) / 128) * cout < limit * 128;
+}
+
 // k = 1, 64-channel steps. 2048 rows, 2048 -> 12288: 103 us on 256 x 192, 109 on 128 x 128, 130 on
 // 128 x 64; 701 rows, 2048 -> 2048: 16 us on 64 x 64, 24 on 128 x 128.
 enum { kTile1_256x256, kTile1_256x192, kTile1_128x128, kTile1_128x64, kTile1_64x64, kTile1Count };

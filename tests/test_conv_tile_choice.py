@@ -51,3 +51,18 @@ def test_narrow_widths_up_to_seven_taps(lanes, length, cin, cout, k, want):
 def test_seven_taps(lanes, length, channels, want):
     assert tile(lanes, length, channels, channels, 7, 3)[:2] == want
     assert split_tile(lanes, length, channels, channels, 7, 3)[:2] == want
+
+
+@pytest.mark.parametrize("lanes,length,cin,cout,want", [
+    # 64 x 64 under the area of 192 tiles of 128 x 128 (128 at 96-multiples)
+    (1, 25, 1536, 6144, (64, 64)), (191, 100, 384, 128, (64, 64)), (1, 9000, 768, 192, (64, 64)),
+    (1, 9000, 384, 320, (64, 64)), (383, 128, 96, 64, (64, 64)), (85, 128, 96, 192, (64, 64)),
+    # the large tiles from there on, register-staged where none divides the width
+    (192, 100, 384, 128, (128, 128)), (4, 2000, 768, 1920, (256, 128)), (86, 128, 96, 192, (128, 96)),
+    (1, 12000, 768, 192, (128, 96)), (384, 128, 96, 64, (256, 64)), (48, 5000, 512, 64, (256, 64)),
+    (1, 12000, 384, 320, (256, 64)), (1, 100, 192, 288, (128, 96)),
+])
+def test_two_taps(lanes, length, cin, cout, want):
+    assert tile(lanes, length, cin, cout, 2)[:2] == want
+    if cout % 96 == 0 or cout % 128 == 0:  # widths the split route takes
+        assert split_tile(lanes, length, cin, cout, 2)[:2] == want
