@@ -142,12 +142,19 @@ auto with_tile(int64_t lanes, int len, int cin, int cout, bool direct, F &&f) {
             if (cout % 128 == 0) return f(Tile<ConvTile<128, 128, 2, 2, 32, KMAX, HMAX, 2, kStageDirect>>{});
             if (cout % 96 == 0) return f(Tile<ConvTile<128, 96, 4, 1, 32, KMAX, HMAX, 2, kStageDirect>>{});
         }
-        // k = 1: 64-channel stages, two (three for the 64 x 64 tile). At few channels and many tiles
-        // the launch moves more bytes than it multiplies: three 32-channel stages and three
-        // workgroups per CU there (24 x 10000 x 384: 123 us, 130 on the 64-channel 128 x 128 tile).
+        // k = 1: 64-channel stages, two (three for the 64 x 64 tile). At fewer than 512 channels a launch moves
+        // more bytes than it multiplies: from 512 tiles of 128 x 128 on three 32-channel stages and three
+        // workgroups per CU (24 x 10000 x 384: 123 us, 130 on the 64-channel 128 x 128 tile); past 384 tiles of
+        // 128 x 64, while 128 x 128 gives fewer or does not divide the width, those (12000 x 384 -> 384: 10.7 us, 11.9 on
+        // 128 x 128, 12.3 on 64 x 64; 72000 x 64 -> 64: 6.6 and 7.4; 20000 x 384 -> 384: 16.3, 14.7 on 128 x 128).
         if constexpr (KMAX == 1) {
-            if (cout % 128 == 0 && cin < 512 && lanes * ((len + 127) / 128) * (cout / 128) >= 1024)
-                return f(Tile<ConvTile<128, 128, 2, 2, 32, KMAX, HMAX, 3, kStageDirect>>{});
+            if (cin < 512 && cout % 64 == 0) {
+                const int64_t rows = lanes * ((len + 127) / 128);
+                const int64_t tiles128 = cout % 128 == 0 ? rows * (cout / 128) : 0;
+                if (tiles128 >= 512) return f(Tile<ConvTile<128, 128, 2, 2, 32, KMAX, HMAX, 3, kStageDirect>>{});
+                if (cin % 64 == 0 && rows * (cout / 64) > 384 && tiles128 < 384)
+                    return f(Tile<ConvTile<128, 64, 2, 2, 64, KMAX, HMAX, 2, kStageDirect>>{});
+            }
             if (cin % 64 == 0) {
                 switch (pick_tile(kTile1, kTile1Count, lanes, len, cout)) {
                     case kTile1_256x256: return f(Tile<ConvTile<256, 256, 2, 4, 64, KMAX, HMAX, 2, kStageDirect>>{});

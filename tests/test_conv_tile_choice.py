@@ -66,3 +66,16 @@ def test_two_taps(lanes, length, cin, cout, want):
     assert tile(lanes, length, cin, cout, 2)[:2] == want
     if cout % 96 == 0 or cout % 128 == 0:  # widths the split route takes
         assert split_tile(lanes, length, cin, cout, 2)[:2] == want
+
+
+@pytest.mark.parametrize("rows,cin,cout,want", [
+    # few channels, many tiles: 32-channel stages, or 128 x 64
+    (40000, 384, 384, (128, 128, 32)), (12000, 384, 384, (128, 64, 64)), (20000, 384, 384, (128, 128, 64)),
+    (72000, 64, 64, (128, 64, 64)), (40000, 192, 192, (128, 64, 64)),
+    # the estimate's five
+    (701, 2048, 2048, (64, 64, 64)), (6400, 768, 768, (128, 64, 64)), (701, 2048, 12288, (256, 192, 64)),
+    (2048, 2048, 4096, (128, 128, 64)), (2048, 6144, 2048, (128, 64, 64)), (3250, 1024, 4096, (256, 256, 64)), (129, 256, 2048, (64, 64, 64)),
+])
+def test_one_tap(rows, cin, cout, want):
+    assert tile(1, rows, cin, cout, 1)[:3] == want
+    assert tile(5, rows // 5, cin, cout, 1)[:3] == tile(1, rows // 5 * 5, cin, cout, 1)[:3]  # the lanes as one sequence
