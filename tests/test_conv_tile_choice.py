@@ -9,6 +9,8 @@ import pytest
 from dtts import lib
 from dtts.nlc import ConvDesc
 
+from test_gpu_conv_tiles import EPILOGUE, ROWS
+
 
 def tile(lanes, length, cin, cout, k, dil=1):
     """(BM, BN, KC, stages, direct staging) of an f16 conv."""
@@ -79,3 +81,22 @@ def test_two_taps(lanes, length, cin, cout, want):
 def test_one_tap(rows, cin, cout, want):
     assert tile(1, rows, cin, cout, 1)[:3] == want
     assert tile(5, rows // 5, cin, cout, 1)[:3] == tile(1, rows // 5 * 5, cin, cout, 1)[:3]  # the lanes as one sequence
+
+
+def _reached(rows):
+    """Per tap class (7, 2, 1) the (BM, BN, KC) of the rows' convs, batched and one lane alone."""
+    out = {7: set(), 2: set(), 1: set()}
+    for lanes, length, cin, cout, k, dil in rows:
+        for n in (lanes, 1):
+            out[k if k <= 2 else 7].add(tile(n, length, cin, cout, k, dil)[:3])
+    return out
+
+
+def test_the_gpu_rows_reach_every_tile():
+    got = _reached(ROWS)
+    assert got[7] >= {(512, 96, 32), (256, 96, 32), (128, 96, 32), (128, 64, 32), (128, 32, 32), (256, 64, 32), (256, 32, 32)}
+    assert got[2] >= {(256, 128, 32), (128, 128, 32), (128, 96, 32), (64, 64, 32), (256, 64, 32)}
+    assert got[1] >= {(256, 256, 64), (256, 192, 64), (128, 128, 64), (128, 64, 64), (64, 64, 64), (128, 128, 32), (128, 96, 32)}
+    got = _reached([(lanes, length, c, c, k, dil) for lanes, length, c, k, dil in EPILOGUE])
+    assert got[7] >= {(512, 96, 32), (256, 96, 32), (128, 96, 32), (128, 64, 32), (128, 32, 32)}
+    assert got[1] >= {(256, 256, 64), (128, 128, 64), (128, 64, 64), (64, 64, 64), (128, 128, 32)}

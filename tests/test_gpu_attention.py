@@ -108,8 +108,8 @@ def test_decode_attention_rejects_bad_arguments(dev):
 
 
 def test_decode_attention_split_past_eight_chunks(dev):
-    """The merge requests up to eight chunks' states at once and loops past that: windows of
-    4700 (ten chunks of 512), 4096 (eight) and 4097 (nine, the last of one position)."""
+    """Windows of 4700 (ten chunks of 512), 4096 (eight) and 4097 (nine, the last of one position), merged
+    in one round."""
     b, n_kv, gqa, cap = 3, 2, 2, 4700
     q, k, v = _inputs(75, b, n_kv, gqa, cap)
     span = np.array([4700, 4096, 4200], np.int32)
@@ -117,3 +117,23 @@ def test_decode_attention_split_past_eight_chunks(dev):
     want = oracle.decode_attention_f32(q, k, v, span, ws)
     split = _run(dev, q, k, v, span, ws)
     assert rel(split, want)[1] < 1e-5
+
+
+@pytest.mark.parametrize("f16", [True, False])
+@pytest.mark.parametrize("gqa,cap,span,ws,peak", [
+    # chunks of 512: sixteen, seventeen (the last of one position), seventeen
+    (2, 8200, (8192, 8193, 8200), (0, 0, 7), (8000, 8192, 8)),
+    # thirty-three, thirty-two, eighteen
+    (1, 16390, (16385, 16384, 8705), (0, 1, 0), (16384, 8192, 4000)),
+])
+def test_decode_attention_many_chunks(dev, f16, gqa, cap, span, ws, peak):
+    """The merge takes up to sixteen chunks' states at once and rescales its sums to a new maximum for the
+    next sixteen: windows on both sides of one and two rounds, the largest score in an early or a late one."""
+    b, n_kv, hd = 3, 2, 64
+    q, k, v = _inputs(75, b, n_kv, gqa, cap, hd, f16)
+    for lane, at in enumerate(peak):  # a score about 6 over the others'
+        row = (60 * q[lane, :, 0]).astype(np.float32)
+        k[lane, :, at] = synth.f16_bits(row) if f16 else row
+    span, ws = np.array(span, np.int32), np.array(ws, np.int32)
+    want = oracle.decode_attention_f32(q, k, v, span, ws)
+    assert rel(_run(dev, q, k, v, span, ws), want)[1] < 1e-5

@@ -1,6 +1,6 @@
-"""The f16 conv's tile choice: every tile of a tap class against float64, at lengths around its tile
-edges, and the same lanes alone and in a batch (another tile, the same bits: all tiles of a class sum
-an output in one order)."""
+"""The f16 conv's tiles: every tile of a tap class against float64, at lengths around its tile edges, and
+the same lanes alone and in a batch (another tile, the same bits: all tiles of a class sum an output in
+one order). That the rows below reach every tile is held in test_conv_tile_choice.py."""
 import pytest
 import torch
 
@@ -43,18 +43,27 @@ def _check(y, ref):
     assert ((y.double() - ref).abs() <= bound).all()
 
 
-@pytest.mark.parametrize("lanes,length,cin,cout,k,dil", [
+# lanes, length, cin, cout, k, dilation
+ROWS = [
     # k <= 7: 128x32, 128x64, 128x96, 256x96, 512x96 and their edges; a run-time tap count
     (1, 1, 64, 96, 7, 1), (1, 25, 1024, 1536, 7, 1), (1, 127, 96, 96, 7, 9), (1, 129, 96, 64, 7, 9), (2, 200, 768, 768, 7, 3),
     (4, 250, 512, 1536, 7, 1), (1, 385, 192, 192, 7, 9), (8, 500, 384, 768, 7, 3), (4, 2001, 384, 768, 7, 3),
     (3, 3000, 384, 384, 7, 9), (24, 1025, 192, 768, 7, 1), (24, 2047, 96, 768, 7, 9), (2, 33, 64, 1024, 3, 1), (3, 511, 32, 32, 5, 2),
+    (24, 501, 96, 192, 7, 9),
+    # ... and the register-staged tiles of widths that are no multiple of 96
+    (170, 100, 64, 64, 5, 1), (170, 257, 32, 32, 3, 2), (30, 701, 64, 160, 7, 9),
     # k = 2: 64x64, 128x128, 256x128, 128x96
     (1, 25, 1536, 6144, 2, 1), (1, 65, 96, 64, 2, 1), (4, 250, 768, 6144, 2, 1), (6, 1000, 768, 1920, 2, 1),
     (1, 1000, 384, 768, 2, 1), (2, 130, 192, 288, 2, 1),
+    (400, 100, 96, 64, 2, 1),
     # k = 1: 64x64, 128x64, 128x128, 256x192, 256x256, 32-channel steps
     (1, 1, 64, 64, 1, 1), (1, 129, 256, 2048, 1, 1), (1, 701, 512, 2048, 1, 1), (5, 411, 512, 2048, 1, 1), (10, 325, 512, 3072, 1, 1),
     (1, 701, 256, 12288, 1, 1), (10, 1300, 512, 1024, 1, 1), (2, 515, 96, 96, 1, 1), (24, 5000, 384, 384, 1, 1), (1, 65, 32, 64, 1, 1),
-])
+    (1, 2043, 512, 4096, 1, 1), (3, 683, 256, 2048, 1, 1),
+]
+
+
+@pytest.mark.parametrize("lanes,length,cin,cout,k,dil", ROWS)
 def test_tiles_against_float64(dev, lanes, length, cin, cout, k, dil):
     x, w, b = _inputs(lanes, length, cin, cout, k, dev)
     y = nlc.conv1d(x, w, b, k=k, dilation=dil)
@@ -63,11 +72,17 @@ def test_tiles_against_float64(dev, lanes, length, cin, cout, k, dil):
     assert torch.equal(alone[0], y[lanes - 1])
 
 
-@pytest.mark.parametrize("lanes,length,k,dil", [(1, 200, 7, 3), (7, 300, 7, 9), (4, 129, 1, 1)])
-def test_small_tiles_epilogue_forms(dev, lanes, length, k, dil):
-    """Residual, both outputs and the SnakeBetas on the tiles that few positions take, against the plain
-    forms composed."""
-    c = 192
+# lanes, length, channels, k, dilation
+EPILOGUE = [
+    (1, 200, 192, 7, 3), (7, 300, 192, 7, 9), (24, 129, 192, 7, 1), (24, 500, 192, 7, 9), (16, 1201, 192, 7, 3), (40, 801, 192, 7, 9),
+    (4, 129, 192, 1, 1), (16, 1201, 192, 1, 1), (24, 300, 512, 1, 1), (16, 1201, 512, 1, 1), (24, 2001, 256, 1, 1),
+]
+
+
+@pytest.mark.parametrize("lanes,length,c,k,dil", EPILOGUE)
+def test_small_tiles_epilogue_forms(dev, lanes, length, c, k, dil):
+    """Residual, both outputs and the SnakeBetas on the tiles that few positions take, and on the larger
+    ones, against the plain forms composed."""
     x, w, b = _inputs(lanes, length, c, c, k, dev)
     act = (torch.rand(c, device=dev) + 0.5, torch.rand(c, device=dev) + 0.5)
     pre, y = nlc.conv1d(x, w, b, k=k, dilation=dil, residual=x, snake_out=act, want_pre=True)

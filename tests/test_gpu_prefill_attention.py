@@ -1,7 +1,8 @@
 """The prefill's 32-query attention blocks at their edges, against the oracle with the prefill's bars
 (outputs 5e-4, written cache entries 1e-3): query counts around a block, key ranges that end inside a
 32-key block of either kind (the cache's rows, the new ones), windows that mask whole blocks for some
-of a block's queries, few and many workgroups."""
+of a block's queries, few and many workgroups. Fewer than 16 queries run on the per-wave kernel, whose
+scores in LDS set its queries per wave and waves per workgroup by the number of keys."""
 from dataclasses import replace
 
 import pytest
@@ -16,12 +17,17 @@ from _util import rel, to_dev, to_host
 pytestmark = pytest.mark.gpu
 
 LONG = replace(SMALL, layers=1, capacity=1024)
+DEEP = replace(LONG, capacity=8200)
 WIN = replace(WINDOWED, layers=1, window=40, capacity=1024)
 
 
 @pytest.mark.parametrize("geo,lanes,t,start", [
     (LONG, 1, 16, 0), (LONG, 2, 31, 1), (LONG, 1, 32, 31), (LONG, 2, 33, 32), (LONG, 1, 65, 33), (LONG, 1, 129, 700),
     (LONG, 1, 500, 0), (WIN, 1, 16, 0), (WIN, 2, 45, 39), (WIN, 1, 100, 41), (WIN, 1, 300, 500), (LONG, 40, 200, 5),
+    # the per-wave kernel: key ranges past one and several strides of 64 lanes, four waves a workgroup (up to
+    # 896 keys), two (up to 1920) and one; four queries a wave (up to 3968 keys), two and one
+    (LONG, 2, 2, 60), (LONG, 1, 3, 64), (LONG, 3, 5, 500), (LONG, 1, 15, 900), (LONG, 2, 2, 127), (WIN, 2, 9, 500),
+    (DEEP, 1, 15, 2000), (DEEP, 1, 6, 4000), (DEEP, 1, 3, 8100),
 ])
 def test_prefill_attention_blocks(dev, geo, lanes, t, start):
     layers, fn = stack.random_weights(geo, 7)

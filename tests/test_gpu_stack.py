@@ -103,7 +103,7 @@ def test_stack_windowed_layer_scale_no_qk_norm(dev):
 
 
 def test_stack_long_cache_splits_attention(dev):
-    """cap 700: windows past 512 positions run as chunks merged by a second launch."""
+    """cap 700: chunks of 128 positions merged by a second launch."""
     geo = replace(SMALL, capacity=700)
     p = Pair(dev, geo, 93, 4, 700)
     p.step(np.array([699, 256, 0, 513], np.int32))
@@ -122,7 +122,7 @@ def test_stack_talker_widths(dev):
 
 
 def test_stack_talker_long_cache_graph_replays(dev):
-    """The talker's widths at its cache capacity (2048): 1-4 chunks per (lane, kv head), spans
+    """The talker's widths at a cache capacity of 2048: 1 to 16 chunks of 128 per (lane, kv head), spans
     ending on and either side of chunk boundaries; an eager step, then graph replays as the
     positions advance."""
     geo = with_layers(replace(stack.TALKER, capacity=2048), 2)

@@ -33,6 +33,8 @@ def edges(lanes, cap, chunk):
     (ONE, "f16", 3, 700, [0, 127, 128]),
     (ONE, "f16", 8, 1600, [0, 1, 255, 256, 511, 512, 1023, 1599]),
     (ONE, "f16", 50, 300, [(i * 37) % 300 for i in range(50)]),
+    # seventeen and thirty-three chunks of 128: the merge in two and three rounds
+    (replace(ONE, capacity=4200), "f16", 2, 4100, [4099, 2048]), (replace(ONE, capacity=4200), "f32", 1, 2049, [2048]),
     (ONE, "q8_0_a32", 2, 1500, [1499, 128]),
     (ONE, "f32", 9, 520, [0, 63, 64, 127, 128, 129, 384, 511, 519]),
     (replace(ONE, n_kv=4), "f16", 2, 400, [399, 200]),  # one query head per kv head
