@@ -138,10 +138,10 @@ int qkrope_apply(const char *name, const float *qkv, const float *norms, const f
     DTTS_REQUIRE((k_f32 == nullptr) == (v_f32 == nullptr), "%s: f32 k and v come together (f32_kv)", name);
     const int64_t waves = b * t * (heads + n_kv);
     DTTS_REQUIRE(waves < (int64_t(1) << 31) && cap < (int64_t(1) << 31), "%s: too many rows", name);
-    qk_rope_span_kernel<float><<<static_cast<unsigned>((waves + 3) / 4), 256, 0, stream>>>(
+    qk_rope_span_kernel<<<static_cast<unsigned>((waves + 3) / 4), 256, 0, stream>>>(
         qkv, norms, cos_t, sin_t, q_out, k_f32, v_f32, reinterpret_cast<half_t *>(kc), reinterpret_cast<half_t *>(vc),
         static_cast<int>(b * t), static_cast<int>(t), static_cast<int>(start), static_cast<int>(heads),
-        static_cast<int>(n_kv), static_cast<int>(hd), static_cast<int>(cap), eps, 1, 0, false);
+        static_cast<int>(n_kv), static_cast<int>(hd), static_cast<int>(cap), eps);
     DTTS_LAUNCH_CHECK(name);
     return DTTS_OK;
 }

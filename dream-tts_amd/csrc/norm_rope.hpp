@@ -218,15 +218,12 @@ __global__ __launch_bounds__(256) void qk_rope_kernel(const T *qkv, const float 
 // QK-norm (when norms is set), RoPE at start + ti and the cache write of t new positions per lane,
 // with the reference's optional f32 side outputs (qkrope::apply with f32_kv, qkrope.rs:26-69):
 // one wave per (row, head), row = bi * t + ti, the lane holding pair (lane, lane + D/2) as the
-// decode kernel does. qkv [rows, (heads + 2 n_kv) D] of T (f32: the sum of ys partials ystride
-// apart, a projection's k-split; f16: the f16 matmul's output). Out: q [b, heads, t, D]; kf and
+// decode kernel does. qkv [rows, (heads + 2 n_kv) D]. Out: q [b, heads, t, D]; kf and
 // vf [b, n_kv, t, D] f32 (both or neither); kc, vc [b, n_kv, cap, D] at start .. start + t - 1.
-template <typename T>
-__global__ __launch_bounds__(256) void qk_rope_span_kernel(const T *qkv, const float *norms, const float *cos_t,
+__global__ __launch_bounds__(256) void qk_rope_span_kernel(const float *qkv, const float *norms, const float *cos_t,
                                                            const float *sin_t, float *q_out, float *kf, float *vf,
                                                            half_t *kc, half_t *vc, int rows, int t, int start, int heads,
-                                                           int n_kv, int hd, int cap, float eps, int ys, int64_t ystride,
-                                                           bool round16) {
+                                                           int n_kv, int hd, int cap, float eps) {
 #pragma clang fp contract(off)
     const int wid = blockIdx.x * 4 + (threadIdx.x >> 6);
     const int lane = threadIdx.x & 63;
@@ -236,26 +233,13 @@ __global__ __launch_bounds__(256) void qk_rope_span_kernel(const T *qkv, const f
     const int h = wid - row * per;
     const int bi = row / t, ti = row - (row / t) * t, p = start + ti;
     const int half = hd / 2;
-    const T *src_row = qkv + static_cast<int64_t>(row) * (heads + 2 * n_kv) * hd;
+    const float *src_row = qkv + static_cast<int64_t>(row) * (heads + 2 * n_kv) * hd;
     const bool is_q = h < heads;
     const bool act = lane < half;
-    auto ld = [&](const T *q) {
-        // the first eight ranges' partials requested together, summed in range order
-        float w[8];
-#pragma unroll
-        for (int y = 0; y < 8; ++y)
-            if (y < ys) w[y] = static_cast<float>(q[y * ystride]);
-        float v = w[0];
-#pragma unroll
-        for (int y = 1; y < 8; ++y)
-            if (y < ys) v += w[y];
-        for (int y = 8; y < ys; ++y) v += static_cast<float>(q[y * ystride]);
-        return round16 ? static_cast<float>(static_cast<half_t>(v)) : v;
-    };
     float x1 = 0.0f, x2 = 0.0f;
     if (act) {
-        x1 = ld(src_row + h * hd + lane);
-        x2 = ld(src_row + h * hd + lane + half);
+        x1 = src_row[h * hd + lane];
+        x2 = src_row[h * hd + lane + half];
     }
     const float ss = wave_sum(x1 * x1 + x2 * x2);
     const float m = sqrtf(ss / static_cast<float>(hd) + eps);
@@ -279,8 +263,8 @@ __global__ __launch_bounds__(256) void qk_rope_span_kernel(const T *qkv, const f
     const int kh = h - heads;
     const int64_t dst = ((static_cast<int64_t>(bi) * n_kv + kh) * cap + p) * hd;
     const int64_t fdst = ((static_cast<int64_t>(bi) * n_kv + kh) * t + ti) * hd;
-    const T *vs = src_row + (heads + n_kv + kh) * hd;
-    const float v1 = ld(vs + lane), v2 = ld(vs + lane + half);
+    const float *vs = src_row + (heads + n_kv + kh) * hd;
+    const float v1 = vs[lane], v2 = vs[lane + half];
     kc[dst + lane] = static_cast<half_t>(o1);
     kc[dst + lane + half] = static_cast<half_t>(o2);
     vc[dst + lane] = static_cast<half_t>(v1);
@@ -293,7 +277,8 @@ __global__ __launch_bounds__(256) void qk_rope_span_kernel(const T *qkv, const f
     }
 }
 
-// The same for the stack's prefill, D in {64, 128} and every operand but norms 16-byte aligned: D/4
+// The same for the stack's prefill, from the QKV projection's output of T (f32: the sum of ys partials
+// ystride apart, a k-split; f16: the f16 matmul's), D in {64, 128}, every operand but norms 16-byte aligned: D/4
 // lanes per (row, head), a lane holding pairs 2j and 2j + 1, so that a wave covers 64 / (D/4) heads with
 // 8-byte f32 and 4-byte f16 accesses (one pair per lane moves half as much per instruction).
 // HBM-bound: 2 (or 4) bytes in and 4 to 6 out per value. 8 x 256 talker positions (59 MB):
