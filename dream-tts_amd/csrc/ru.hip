@@ -303,8 +303,8 @@ __global__ __launch_bounds__(Cfg::THREADS, Cfg::WPE) void ru_nlc_f16(RuArgs q) {
             // before the last tap's MFMAs: every wave then has this chunk's last fragments in
             // registers, and the next chunk's first ones are read under those MFMAs. With the window
             // unpadded (its writes took 16 LDS cycles each padded, 13 now) and the reads spread between
-            // the MFMAs: 16 x 40000 x 192, 514 -> 507 us; the chip's power limit takes the rest (the
-            // tile alone: 36.7 -> 33.9 us).
+            // the MFMAs a tile alone takes 33.9 us instead of 36.7, 16 x 40000 x 192 1% to 2.5% less (526 -> 521,
+            // 486 -> 475 us in separate runs).
 #pragma unroll
             for (int t = 0; t < KT; ++t) {
                 const int set = (c * KT + t) & 1;

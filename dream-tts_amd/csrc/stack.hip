@@ -699,9 +699,11 @@ __global__ __launch_bounds__(256) void prefill_attention(const float *q, const h
 // output block db is dimension NDB r + db, so a lane reads its dimensions of a value row in one load.
 // K's next block loads under P . V, V's under K . Q^T.
 //
-// Bound: the f32 matrix rate, 2 D / 64 MFMAs of 64 cycles per wave and block, and the longest
-// workgroup of a causal block row (long rows are dispatched first). Talker prompts, per layer: 1 x 701
-// (352 workgroups) 166 us on prefill_attention -> 53, 8 x 256 (1024) 74 us with the scores in LDS -> 50.
+// Work: D MFMAs of 64 cycles per wave and block (half for the scores, half for P . V), 16 us of the chip a
+// talker layer at 1 x 701 and at 8 x 256; it takes 55 and 53, a third of that rate: the longest workgroup
+// of a causal block row (long rows are dispatched first), CUs with a long and a short one, the softmax
+// between the MFMAs. Before: 1 x 701 (352 workgroups) 166 us on prefill_attention, 8 x 256 (1024) 74 us with
+// the scores in LDS.
 constexpr int kPrefillFlashMinT = 16;  // fewer queries leave most of a 32-query block idle
 // Waves per workgroup, the same for every launch: the count is the order in which a query's keys are summed,
 // and a prompt's result does not depend on the prompts beside it. With two waves a one-layer talker prompt
