@@ -114,15 +114,25 @@ __device__ __forceinline__ float softmax_exp2(float x) { return __builtin_amdgcn
 
 // Positions per workgroup when a span is split: kChunk at the entry points, whose workspace sizes
 // are part of their interface. The stack step, which owns its workspace, halves it down to kChunkMin
-// while the launch has fewer than three workgroups per CU: a workgroup is a chain of dependent
-// softmax updates, and few lanes leave most CUs without one. 8 lanes, f32 caches of 1536 positions:
-// 28.8 -> 15.3 us a layer, the merge 4.8 -> 5.3.
+// while the launch has few workgroups: a workgroup is a chain of dependent softmax updates, and few lanes
+// leave most CUs without one (8 lanes, f32 caches of 1536 positions: 28.8 -> 15.3 us a layer, the merge
+// 4.8 -> 5.3). Lines from 1 to 64 lanes and 64 to 4000 positions at 1, 2, 4 and 8 query heads per kv head:
+// - fewer than kChunkFill workgroups (three per CU); 512 for f16 caches at 1 or 4 query heads, 320 at 8, whose
+//   workgroups each combine 16 position groups of 8 heads (2 kv heads, D = 128, two layers: 64 lanes x 600
+//   positions 14% faster at 384 workgroups than at 256; 16 lanes x 4000, the worst, 156 us at 256, 167 at 512, 225
+//   at 1024);
+// - at most 128 chunks x query heads, the rows that a merging workgroup reads;
+// - a window that a merge costs more than it gives stays whole: 320 positions, 256 with f32 caches (32 lanes x 8 kv
+//   heads x 300 positions, f16, one query head: 90.5 us whole, 94.5 in two chunks).
 constexpr int kChunk = 512, kChunkMin = 128, kChunkFill = 768;
 
-inline int attn_step_chunk(int64_t b, int64_t n_kv, int64_t max_window) {
+inline int attn_step_chunk(int64_t b, int64_t n_kv, int64_t gqa, bool f32, int64_t max_window) {
+    if (max_window <= (f32 && gqa < 8 ? 256 : 320)) return kChunk;
+    const int64_t fill = gqa >= 8 ? 320 : gqa == 2 || f32 ? kChunkFill : 512;
+    auto chunks = [&](int c) { return (max_window + c - 1) / c; };
     int c = kChunk;
-    while (c > kChunkMin && b * n_kv * ((max_window + c - 1) / c) < kChunkFill) c /= 2;
-    return c < 2 * kChunkMin && max_window <= 2 * kChunkMin ? 2 * kChunkMin : c;  // a short window stays whole
+    while (c > kChunkMin && b * n_kv * chunks(c) < fill && chunks(c / 2) * gqa <= 128) c /= 2;
+    return c;
 }
 
 // Chunks of a lane's window [lo, hi) when split; a chunk is a power of two.
@@ -134,14 +144,18 @@ __device__ __host__ inline int chunks_of(int lo, int hi, int chunk) {
 // arithmetic as qk_rope_kernel): each makes its kv head's queries from the QKV projection's output,
 // and the one whose chunk holds the new position also makes its k and v rows and writes the caches.
 // Every chunk's workgroup repeats its GQA query rows of D values, which come from L2; the launch and its
-// gap are gone (a predictor step at one lane 181 -> 169 us). Up to kStepFuseMax (lane, kv head) pairs it
-// is the faster way at every window (two talker layers, f16 caches of 1536: 1 lane 111 -> 104.5 us, 16
-// lanes 140.3 -> 133.3), and beyond them while a window has at most two chunks (48 lanes: 257 positions
-// 142 -> 129 us, 800 6% to 12%, a predictor's 17 204 -> 191). With three chunks or more and more pairs it is
-// between 14% faster and 2% slower (48 lanes of 1536: 200.3 -> 202.0), and qk_rope_kernel stays.
+// gap are gone (a predictor step at one lane 181 -> 169 us). With one or two query heads per kv head it is
+// the faster way at every window up to kStepFuseMax (lane, kv head) pairs (two talker layers, f16 caches of
+// 1536: 1 lane 111 -> 104.5 us, 16 lanes 140.3 -> 133.3), and beyond them while a window has at most two chunks (48
+// lanes: 257 positions 142 -> 129 us, 800 6% to 12%, a predictor's 17 204 -> 191). With three chunks or more and
+// more pairs it is between 14% faster and 2% slower (48 lanes of 1536: 200.3 -> 202.0), and qk_rope_kernel stays.
+// Four query heads: from two chunks on (one: 2% to 6% slower). Eight, ten rows for four waves: 5% to 25%
+// slower at most sizes, never.
 constexpr int kStepFuseMax = 128;
 
-inline bool step_fuses(int64_t pairs, int64_t chunks) { return pairs <= kStepFuseMax || chunks <= 2; }
+inline bool step_fuses(int64_t pairs, int64_t gqa, int64_t chunks) {
+    return gqa <= 4 && (gqa < 4 || chunks > 1) && (pairs <= kStepFuseMax || chunks <= 2);
+}
 
 struct QkvStep {
     const float *qkv;      // [b, (heads + 2 n_kv) D], or ys partials of it `stride` floats apart
@@ -487,7 +501,7 @@ hipError_t launch_gqa(const float *q, T *kc, T *vc, OutT *out, float *part, int 
     return hipGetLastError();
 }
 
-// gqa in {1, 2, 4, 8} and D in {64, 128}, checked by the caller.
+// gqa in {1, 2, 4, 8} (8: NoStep only) and D in {64, 128}, checked by the caller.
 template <typename T, typename Src, typename OutT, typename Step>
 hipError_t launch_attention(const float *q, T *kc, T *vc, OutT *out, float *part, int max_window,
                             int chunk, int64_t b, int64_t n_kv, int64_t gqa, int64_t head_dim, int64_t cap, const Src &sp,
@@ -498,14 +512,20 @@ hipError_t launch_attention(const float *q, T *kc, T *vc, OutT *out, float *part
             case 1: return launch_gqa<T, 128, 1>(q, kc, vc, out, part, max_chunks, chunk, b, n_kv, cap, sp, st, stream);
             case 2: return launch_gqa<T, 128, 2>(q, kc, vc, out, part, max_chunks, chunk, b, n_kv, cap, sp, st, stream);
             case 4: return launch_gqa<T, 128, 4>(q, kc, vc, out, part, max_chunks, chunk, b, n_kv, cap, sp, st, stream);
-            default: return launch_gqa<T, 128, 8>(q, kc, vc, out, part, max_chunks, chunk, b, n_kv, cap, sp, st, stream);
+            default:
+                if constexpr (std::is_same<Step, NoStep>::value)
+                    return launch_gqa<T, 128, 8>(q, kc, vc, out, part, max_chunks, chunk, b, n_kv, cap, sp, st, stream);
+                return hipErrorInvalidValue;
         }
     }
     switch (gqa) {
         case 1: return launch_gqa<T, 64, 1>(q, kc, vc, out, part, max_chunks, chunk, b, n_kv, cap, sp, st, stream);
         case 2: return launch_gqa<T, 64, 2>(q, kc, vc, out, part, max_chunks, chunk, b, n_kv, cap, sp, st, stream);
         case 4: return launch_gqa<T, 64, 4>(q, kc, vc, out, part, max_chunks, chunk, b, n_kv, cap, sp, st, stream);
-        default: return launch_gqa<T, 64, 8>(q, kc, vc, out, part, max_chunks, chunk, b, n_kv, cap, sp, st, stream);
+        default:
+            if constexpr (std::is_same<Step, NoStep>::value)
+                return launch_gqa<T, 64, 8>(q, kc, vc, out, part, max_chunks, chunk, b, n_kv, cap, sp, st, stream);
+            return hipErrorInvalidValue;
     }
 }
 
@@ -519,8 +539,8 @@ inline size_t attn_workspace_bytes(int64_t b, int64_t n_kv, int64_t gqa, int64_t
 
 // The stack step's workspace: room for every window up to max_window at any lane count up to b, so that
 // one sized for the largest batch and capacity serves the smaller ones, whose chunks are shorter (a chunk
-// below kChunk is taken only while twice its length gives under kChunkFill workgroups, so its chunks stay
-// under twice the filling count). From kChunkFill lanes on the need only grows with the lanes.
+// below kChunk is taken only while twice its length gives under kChunkFill workgroups at most, so its chunks
+// stay under twice the filling count). From kChunkFill lanes on the need only grows with the lanes.
 inline size_t attn_step_workspace_bytes(int64_t b, int64_t n_kv, int64_t gqa, int64_t head_dim, int64_t max_window) {
     if (b <= 0 || n_kv <= 0 || gqa <= 0 || head_dim <= 0 || max_window <= 2 * kChunkMin) return 0;
     const int64_t shortest = (max_window + kChunkMin - 1) / kChunkMin, longest = (max_window + kChunk - 1) / kChunk;

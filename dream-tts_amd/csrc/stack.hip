@@ -216,7 +216,7 @@ Plan plan_of(const dtts_stack_geometry &g, int64_t lanes, int64_t cap) {
     p.gemm_part = take(gb);
     const int64_t win = g.window > 0 && g.window < cap ? g.window : cap;
     p.max_window = static_cast<int>(win);
-    p.attn_chunk = attn_step_chunk(lanes, g.n_kv, win);
+    p.attn_chunk = attn_step_chunk(lanes, g.n_kv, g.heads / g.n_kv, false, win);
     p.attn_bytes = attn_step_workspace_bytes(lanes, g.n_kv, g.heads / g.n_kv, g.head_dim, win);
     p.attn_part = take(p.attn_bytes);
     p.total = off;
@@ -266,7 +266,7 @@ hipError_t step_attention(const dtts_stack &s, const dtts_stack_layer &L, T *kc,
     const float *norms = g.qk_norm ? L.qk_norms : nullptr;
     const float qscale = g.qk_norm ? 1.0f : static_cast<float>(1.0 / std::sqrt(static_cast<double>(g.head_dim)));
     const DevSpans spans{s.pos, static_cast<int>(g.window)};
-    if (step_fuses(lanes * n_kv, part ? (max_window + chunk - 1) / chunk : 1)) {
+    if (step_fuses(lanes * n_kv, heads / n_kv, part ? (max_window + chunk - 1) / chunk : 1)) {
         const QkvStep st{qkv.p, qkv.ys, qkv.stride, round16, norms, s.cos_t, s.sin_t, g.eps, qscale};
         return launch_attention(nullptr, kc, vc, out, part, max_window, chunk, lanes, n_kv, heads / n_kv, hd, cap, spans, st,
                                 stream);
@@ -413,7 +413,7 @@ PlanW plan_w(const dtts_stack_geometry &g, int32_t how, int64_t lanes, int64_t c
     p.part = take(pb);
     const int64_t win = g.window > 0 && g.window < cap ? g.window : cap;
     p.max_window = static_cast<int>(win);
-    p.attn_chunk = attn_step_chunk(lanes, g.n_kv, win);
+    p.attn_chunk = attn_step_chunk(lanes, g.n_kv, g.heads / g.n_kv, true, win);
     p.attn_bytes = attn_step_workspace_bytes(lanes, g.n_kv, g.heads / g.n_kv, g.head_dim, win);
     p.attn_part = take(p.attn_bytes);
     p.total = off;

@@ -1,7 +1,7 @@
 """The decode step at few lanes against the oracle, where its attention splits spans into shorter chunks:
 positions on both sides of a chunk's edge, one lane to the batch that fills the chip, both cache types,
-grouped heads and windows, on both sides of the line to which the attention makes its own q, k and v
-(128 (lane, kv head) pairs, or two chunks). Bars as test_gpu_stack.py's."""
+grouped heads and windows, on both sides of the lines to which the attention makes its own q, k and v
+(128 (lane, kv head) pairs, or two chunks; up to four query heads per kv head). Bars as test_gpu_stack.py's."""
 from dataclasses import replace
 
 import numpy as np
@@ -29,7 +29,9 @@ def edges(lanes, cap, chunk):
 
 @pytest.mark.parametrize("geo,weight,lanes,cap,pos", [
     (ONE, "f16", 1, 256, [255]),                      # one chunk
-    (ONE, "f16", 1, 257, [256]),                      # three chunks, the last of one position
+    (ONE, "f16", 1, 257, [256]), (ONE, "f16", 1, 320, [319]),  # still one
+    (ONE, "f16", 1, 321, [320]), (ONE, "f32", 1, 257, [256]),  # three of 128, the last of 65 and of one position
+    (ONE, "f16", 1, 385, [384]),                      # four, the last of one
     (ONE, "f16", 3, 700, [0, 127, 128]),
     (ONE, "f16", 8, 1600, [0, 1, 255, 256, 511, 512, 1023, 1599]),
     (ONE, "f16", 50, 300, [(i * 37) % 300 for i in range(50)]),
@@ -39,10 +41,15 @@ def edges(lanes, cap, chunk):
     (ONE, "f32", 9, 520, [0, 63, 64, 127, 128, 129, 384, 511, 519]),
     (replace(ONE, n_kv=4), "f16", 2, 400, [399, 200]),  # one query head per kv head
     (replace(ONE, heads=8, n_kv=1, head_dim=64), "f16", 2, 400, [399, 129]),  # eight
+    (replace(ONE, heads=8, n_kv=1), "f32", 3, 700, [699, 384, 5]), (replace(ONE, heads=8, n_kv=1), "f16", 2, 64, [63, 0]),
+    # four: in the attention's launch from two chunks on
+    (replace(ONE, heads=8), "f16", 2, 64, [63, 0]), (replace(ONE, heads=8), "f16", 3, 700, [699, 384, 5]),
+    (replace(ONE, heads=8, head_dim=64), "f32", 3, 1500, [1499, 128, 127]), (replace(ONE, heads=8), "f32", 2, 200, [199, 1]),
     (replace(WINDOWED, layers=1, window=300, capacity=700), "f16", 4, 700, [10, 299, 300, 699]),
+    (replace(WINDOWED, layers=1, window=400, capacity=700), "f16", 4, 700, [10, 399, 400, 699]),
     # more than 128 pairs: three chunks or more after the qk-rope kernel, up to two without it
-    (EIGHT, "f16", 17, 1100, edges(17, 1100, 128)), (EIGHT, "f32", 17, 1100, edges(17, 1100, 128)),
-    (EIGHT, "f16", 24, 1100, edges(24, 1100, 256)), (EIGHT, "f32", 33, 600, edges(33, 600, 256)),
+    (replace(EIGHT, heads=16), "f16", 17, 1100, edges(17, 1100, 128)), (EIGHT, "f32", 17, 1100, edges(17, 1100, 128)),
+    (EIGHT, "f16", 17, 1100, edges(17, 1100, 256)), (EIGHT, "f32", 33, 600, edges(33, 600, 256)),
     (EIGHT, "f16", 48, 1536, edges(48, 1536, 512)), (EIGHT, "f32", 48, 1025, edges(48, 1025, 512)),
     (replace(EIGHT, heads=16, head_dim=128), "f16", 24, 1100, edges(24, 1100, 256)),
     (replace(WINDOWED, layers=1, heads=8, n_kv=8, window=700, capacity=1100), "f16", 24, 1100, edges(24, 1100, 256)),
